@@ -183,6 +183,7 @@ static st_status resolve(const st_params *p, Cfg &c, bool mixed)
     c.rowc = 0;
     c.wy_d = c.core_d = c.zchunk_d = c.lds_d = 0;
     c.shell_eq = nullptr;
+    c.block_steps = 0;
     c.zchunk = 0;
     c.lds = 0;
     c.gx = c.gy = c.gz = 1;
@@ -239,6 +240,9 @@ static st_status resolve(const st_params *p, Cfg &c, bool mixed)
             c.variant = march_ok ? ST_V_SMEM_REGISTER : ST_V_BASE;
             if (!march_ok) c.cx = 1;
         }
+        // 2D grids of radius 1 fuse sweeps per launch whichever family the
+        // rules above name (that family still serves stencil_sweep)
+        if (c.form == 0 && p->temporal_steps == 0) resolve_block(c);
     }
     switch (c.variant) {
     case ST_V_BASE: return resolve_base(c);
@@ -320,6 +324,10 @@ st_status stencil_launch_config(const st_params *p, st_launch_info *info)
         } else {
             info->launches = c.iters;
         }
+        if (c.block_steps) {
+            info->temporal_steps = c.block_steps;
+            info->launches = block_launches(c);
+        }
     }
     return ST_OK;
 }
@@ -352,7 +360,9 @@ st_status stencil_dispatch(const st_params *p, void *d_u1, void *d_u2, void *str
     }
     {
         int in_u2 = 0;
-        if (c.variant == ST_V_COOP) {
+        if (c.block_steps) {
+            s = run_block(c, d_u1, d_u2, hs, &in_u2);
+        } else if (c.variant == ST_V_COOP) {
             s = run_coop(c, d_u1, d_u2, hs, &in_u2);
         } else {
             // the row form stores whole rows when both shells are equal

@@ -37,6 +37,40 @@ __device__ __forceinline__ T finish(T sum, T centre, T kc)
     }
 }
 
+// finish() of N sums whose chain starts with the first neighbour instead of
+// 0 + it: the two differ only where every neighbour is -0 (the chain from 0
+// is never -0), and the FMA with +0 (JACOBI) and the quotient below (THESIS)
+// give +0 there as well.
+//
+// The THESIS quotient sum / kc (kc a small whole number) is corrected from a
+// multiplication by the rounded reciprocal: q = sum*rk, q + (sum - kc*q)*rk
+// with both steps fused is the correctly rounded quotient (Markstein, IBM J.
+// Res. Dev. 34(1), 1990) as long as q is zero or normal: a tie, which only a
+// subnormal quotient can be, and infinities and NaN take the division.  Three
+// operations and a class test instead of the eleven of the division.
+template <int OP, int N, typename T>
+__device__ __forceinline__ void finish_sums(const T (&sum)[N], const T (&centre)[N], T kc, T (&out)[N])
+{
+    if constexpr (OP == OP_THESIS) {
+        const T rk = (T)1 / kc;
+        bool odd = false;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const T q = sum[i] * rk;
+            odd |= __builtin_isfpclass(q, 0x0003 | 0x0204 | 0x0090);  // NaN, +-infinity, +-subnormal
+            const T e = __builtin_elementwise_fma(-kc, q, sum[i]);
+            out[i] = __builtin_elementwise_fma(e, rk, q) - centre[i];
+        }
+        if (__builtin_expect(__any(odd), 0)) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) out[i] = (sum[i] + (T)0) / kc - centre[i];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) out[i] = __builtin_elementwise_fma(sum[i], kc, (T)0);
+    }
+}
+
 __device__ __forceinline__ bool interior1(int i, int n, int r) { return i >= r && i < n - r; }
 
 // Cross-lane read of a 32-bit or 64-bit value from lane `src` (0..63; any

@@ -33,6 +33,7 @@ struct Cfg {
     int rowc;            // row form: 1 = consecutive columns per lane (k_rowc)
     int wy_d, core_d;    // COOP streaming form, kernel for different shells (when its
     int zchunk_d, lds_d; // frame differs): wave rows, core rows, z chunk, LDS bytes
+    int block_steps;     // AUTO: sweeps per launch of the block form (0: not used)
     const int *shell_eq; // device flag: both buffers' shells hold the same bits
                          // (row form stores whole rows then); null: unknown
 };
@@ -90,6 +91,13 @@ bool rows_mixed_fused_ok(const Cfg &c);
 // shell); without, x' = x and x_out is unused.
 st_status launch_rows_defect(const Cfg &c, bool f16, const float *x, const uint16_t *e_old, float *x_out,
                              uint16_t *d, uint16_t *e_first, hipStream_t s);
+
+// Block form, several sweeps of a register-resident block per launch
+// (sweep_block.hip), for the dispatches that AUTO gives it; both buffers end
+// as single sweeps leave them.
+void resolve_block(Cfg &c);        // sets c.block_steps (0 where it is not taken)
+int block_launches(const Cfg &c);
+st_status run_block(const Cfg &c, void *u1, void *u2, hipStream_t s, int *in_u2);
 
 // 2D streaming temporal blocking, four or six fused sweeps per pass
 // (sweep_stream2d.hip); `single` is the per-sweep configuration for the
