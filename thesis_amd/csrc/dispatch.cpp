@@ -49,7 +49,7 @@ st_status hip_check(hipError_t e, const char *what)
 // share device scratch (shell flags, reduction partials, batch tables), and
 // calls on one stream are ordered by the stream.
 static std::mutex g_ws_mutex;
-constexpr int kSlots = 4;
+constexpr int kSlots = 5;
 struct WsBlock {
     void *ptr = nullptr;
     size_t size = 0;
@@ -63,10 +63,12 @@ static thread_local const WsFixed *g_ws_fixed = nullptr;
 void workspace_use_fixed(const WsFixed *fixed) { g_ws_fixed = fixed; }
 bool workspace_is_fixed() { return g_ws_fixed != nullptr; }
 
-st_status workspace_slot(int slot, size_t bytes, hipStream_t stream, void **ptr)
+st_status workspace_slot(int slot, size_t bytes, hipStream_t stream, void **ptr, size_t *fresh)
 {
+    if (fresh) *fresh = 0;
     if (slot < 0 || slot >= kSlots) return fail(ST_EINVAL, "workspace slot %d", slot);
     if (g_ws_fixed) {
+        if (slot >= 4) return fail(ST_EINVAL, "workspace slot %d has no fixed part", slot);
         const size_t part = g_ws_fixed->bytes[slot];
         if (bytes > part)
             return fail(ST_EINVAL, "workspace of %zu bytes exceeds the fixed scratch part of %zu bytes (slot %d)",
@@ -89,9 +91,14 @@ st_status workspace_slot(int slot, size_t bytes, hipStream_t stream, void **ptr)
             w.size = 0;
         }
         size_t sz = bytes < (1u << 20) ? (1u << 20) : bytes;
+        // another stream of this thread may be under capture
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
         e = hipMalloc(&w.ptr, sz);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
         if (e != hipSuccess) return hip_check(e, "workspace hipMalloc");
         w.size = sz;
+        if (fresh) *fresh = sz;
     }
     *ptr = w.ptr;
     return ST_OK;
@@ -184,6 +191,7 @@ static st_status resolve(const st_params *p, Cfg &c, bool mixed)
     c.wy_d = c.core_d = c.zchunk_d = c.lds_d = 0;
     c.shell_eq = nullptr;
     c.block_steps = 0;
+    c.resident = 0;
     c.zchunk = 0;
     c.lds = 0;
     c.gx = c.gy = c.gz = 1;
@@ -242,7 +250,11 @@ static st_status resolve(const st_params *p, Cfg &c, bool mixed)
         }
         // 2D grids of radius 1 fuse sweeps per launch whichever family the
         // rules above name (that family still serves stencil_sweep)
-        if (c.form == 0 && p->temporal_steps == 0) resolve_block(c);
+        if (c.form == 0 && p->temporal_steps == 0) {
+            resolve_block(c);
+            // small 3D grids of radius 1: every sweep in one launch
+            c.resident = resident_eligible(c, 1);
+        }
     }
     switch (c.variant) {
     case ST_V_BASE: return resolve_base(c);
@@ -328,6 +340,10 @@ st_status stencil_launch_config(const st_params *p, st_launch_info *info)
             info->temporal_steps = c.block_steps;
             info->launches = block_launches(c);
         }
+        if (c.resident) {
+            info->temporal_steps = c.iters;
+            info->launches = 1;
+        }
     }
     return ST_OK;
 }
@@ -360,7 +376,15 @@ st_status stencil_dispatch(const st_params *p, void *d_u1, void *d_u2, void *str
     }
     {
         int in_u2 = 0;
-        if (c.block_steps) {
+        bool done = false;
+        if (c.resident) {
+            void *u[1][2] = {{d_u1, d_u2}};
+            s = run_resident(c, 1, u, hs, &done);
+            in_u2 = c.iters & 1;
+        }
+        if (done || s != ST_OK) {
+            // done, or failed
+        } else if (c.block_steps) {
             s = run_block(c, d_u1, d_u2, hs, &in_u2);
         } else if (c.variant == ST_V_COOP) {
             s = run_coop(c, d_u1, d_u2, hs, &in_u2);

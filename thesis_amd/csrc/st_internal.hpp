@@ -33,6 +33,7 @@ struct Cfg {
     int rowc;            // row form: 1 = consecutive columns per lane (k_rowc)
     int wy_d, core_d;    // COOP streaming form, kernel for different shells (when its
     int zchunk_d, lds_d; // frame differs): wave rows, core rows, z chunk, LDS bytes
+    int resident;        // AUTO: the resident form runs the dispatch
     int block_steps;     // AUTO: sweeps per launch of the block form (0: not used)
     const int *shell_eq; // device flag: both buffers' shells hold the same bits
                          // (row form stores whole rows then); null: unknown
@@ -99,6 +100,13 @@ void resolve_block(Cfg &c);        // sets c.block_steps (0 where it is not take
 int block_launches(const Cfg &c);
 st_status run_block(const Cfg &c, void *u1, void *u2, hipStream_t s, int *in_u2);
 
+// Resident form, every sweep in one cooperative launch with the field in
+// registers (sweep_resident.hip), on `problems` grids of the same shape; both
+// buffers end as single sweeps leave them.  *done false: not launched (no
+// cooperative launch now, a stream under capture, or no allocation allowed).
+bool resident_eligible(const Cfg &c, int problems);
+st_status run_resident(const Cfg &c, int problems, void *const (*u)[2], hipStream_t s, bool *done);
+
 // 2D streaming temporal blocking, four or six fused sweeps per pass
 // (sweep_stream2d.hip); `single` is the per-sweep configuration for the
 // sweeps outside fused passes.
@@ -121,7 +129,10 @@ st_status run_mixed(const Cfg &c, void *x, void *e1, void *e2, void *d, void *u,
 
 // Library-owned device workspace (grows on demand, one per device, stream
 // and slot).
-st_status workspace_slot(int slot, size_t bytes, hipStream_t stream, void **ptr);
+// *fresh (optional) receives the block's size when this call allocated it,
+// else 0.
+st_status workspace_slot(int slot, size_t bytes, hipStream_t stream, void **ptr, size_t *fresh = nullptr);
+constexpr int kSlotResident = 4;  // the resident form's own slot (its contents last from call to call)
 // A fixed device buffer that serves every workspace request of the calling
 // thread while it is set (one part per slot; a request larger than its
 // slot's part fails with ST_EINVAL); null returns to the allocated
