@@ -14,10 +14,14 @@
 //
 // The backward data pass is the same kernel applied to the gradient with
 // the weights transposed and the taps mirrored (conv_wt_transpose); the
-// weight gradient is a second MFMA GEMM reducing over positions with float
-// atomics into FP32.
+// weight gradient is a second MFMA GEMM reducing over positions.  Both take
+// their operands from tiles staged in LDS (k_conv3_tile, k_conv3_wgrad_tile);
+// k_conv3 and k_conv3_wgrad, which load every operand from global memory,
+// serve the shapes whose tile does not fit.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <algorithm>
 
 #include "../../include/stencil_nn.h"
 #include "st_device.hpp"
@@ -36,6 +40,15 @@ __device__ __forceinline__ bf16_t f2bf(float f)
     if ((x & 0x7fffffffu) > 0x7f800000u) return (bf16_t)((x >> 16) | 0x40);
     x += 0x7fffu + ((x >> 16) & 1u);
     return (bf16_t)(x >> 16);
+}
+
+// two values rounded to BF16, low word first (v_cvt_pk_bf16_f32: round to
+// nearest even, the same words as f2bf)
+__device__ __forceinline__ uint32_t pack_bf(float a, float b)
+{
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const bf16x2 v = {(__bf16)a, (__bf16)b};
+    return __builtin_bit_cast(uint32_t, v);
 }
 
 __device__ __forceinline__ float bf2f(bf16_t h) { return __uint_as_float((uint32_t)h << 16); }
@@ -179,6 +192,224 @@ __global__ __launch_bounds__(256) void k_conv3(const bf16_t *__restrict__ act,
     }
 }
 
+// ---------------------------------------------------------------- conv forward / backward data, LDS tiles
+
+// The same sums in the same order (chunks of 32 weight columns, one MFMA
+// each), with the activations read from LDS: a workgroup of four waves stages
+// the 18 x 6 x (TZ+2) neighbourhood of a tile of 16 x 4 x TZ positions once
+// and takes all 27 taps from it, where k_conv3 loads every operand of every
+// tap from global memory (16 bytes per lane and MFMA: the L2 and its address
+// arithmetic held it at 180 TFLOP/s).  A wave computes MB rows of 16
+// positions and 16*NB output channels.
+//
+// Bound: LDS reads (1 KiB per wave and MFMA at NB = 1; a CU reads 128 bytes
+// a cycle and starts an MFMA every 4) and the staging of the tiles, which two
+// workgroups per CU overlap in part.  8 x 64^3 positions, k_conv3 and now:
+// 48 -> 16 channels 453 -> 272 us, 16 -> 48 FP32 489 -> 266, 16 -> 16 159 ->
+// 92; 8 x 16^3, 64 -> 64 64 -> 31.  Weights straight from L2 (16 rows of 64
+// bytes per load) instead of through LDS: 16 -> 48 370 us.  The position
+// stride in LDS carries 16 bytes of padding where Ci is a multiple
+// of 32, else eight lanes of a read would meet in the same banks.
+constexpr int kTx = 16, kTy = 4;
+
+// LDS bytes from one position of a tile to the next
+__host__ __device__ constexpr int tile_stride(int ci) { return 2 * (ci % 32 == 0 ? ci + 8 : ci); }
+__host__ __device__ constexpr int tile_positions(int tz) { return (kTx + 2) * (kTy + 2) * (tz + 2); }
+
+struct TileGeom {
+    ConvGeom g;
+    int tx, ty, tz;  // tiles per axis (of one sample)
+};
+
+// Tile `t`: sample and first position.
+__device__ __forceinline__ void tile_origin(const TileGeom &q, int t, int depth, int &n, int &z, int &y, int &x)
+{
+    x = t % q.tx * kTx;
+    t /= q.tx;
+    y = t % q.ty * kTy;
+    t /= q.ty;
+    z = t % q.tz * depth;
+    n = t / q.tz;
+}
+
+// Stage the neighbourhood of a tile of depth TZ (positions -1 .. +1 around
+// it; zero outside the sample): all Ci channels, position stride S bytes.
+// A row of 18 positions is one run of memory; a wave takes a row at a time in
+// 16-byte words, so the words' places are computed once per wave (computing
+// them per word took as many instructions as the products).
+template <int TZ, int WAVES>
+__device__ __forceinline__ void tile_stage(const bf16_t *__restrict__ act, const ConvGeom &g, int n, int z0, int y0,
+                                           int x0, char *lds, int S)
+{
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nc8 = g.Ci >> 3, words = (kTx + 2) * nc8;
+    const long long sample = (long long)n * g.D * g.H * g.W;
+    constexpr int ROWS = (kTy + 2) * (TZ + 2);
+    for (int i0 = 0; i0 < words; i0 += 64) {
+        const int i = i0 + lane, px = i / nc8, c8 = i - px * nc8;
+        const bool have = i < words, xin = have && (unsigned)(x0 + px - 1) < (unsigned)g.W;
+        const unsigned go = (unsigned)i * 16u;  // byte offset in the row, from position x0 - 1
+        char *const to = lds + px * S + c8 * 16;
+#pragma unroll 5
+        for (int r = w; r < ROWS; r += WAVES) {
+            const int py = r % (kTy + 2), pz = r / (kTy + 2), y = y0 + py - 1, z = z0 + pz - 1;
+            const bool rin = (unsigned)y < (unsigned)g.H && (unsigned)z < (unsigned)g.D;
+            u32x4 v = {0u, 0u, 0u, 0u};
+            if (rin && xin) {
+                const char *row = reinterpret_cast<const char *>(act + (sample + ((long long)z * g.H + y) * g.W + x0 - 1) * g.Ci);
+                v = *reinterpret_cast<const u32x4 *>(row + go);
+            }
+            if (have) *reinterpret_cast<u32x4 *>(to + r * (kTx + 2) * S) = v;
+        }
+    }
+}
+
+// LDS offset of tap `tap`, channel `ci`, from a position's first neighbour
+__device__ __forceinline__ int tap_offset(int tap, int ci, int S)
+{
+    return ((tap / 9 * (kTy + 2) + tap / 3 % 3) * (kTx + 2) + tap % 3) * S + 2 * ci;
+}
+
+// weight chunks staged at a time
+__host__ __device__ constexpr int conv_chunks(int nb) { return nb == 1 ? 8 : 4; }
+
+template <int NB, int MB>
+__global__ __launch_bounds__(256) void k_conv3_tile(const bf16_t *__restrict__ act, const bf16_t *__restrict__ wt,
+                                                    const float *__restrict__ bias, bf16_t *__restrict__ out_bf,
+                                                    float *__restrict__ out_f, TileGeom q, int nct, int relu,
+                                                    int accumulate)
+{
+    constexpr int TZ = MB;  // 4*MB rows of 16 positions, MB per wave
+    constexpr int KC = conv_chunks(NB), WR = KC * NB / 4;
+    extern __shared__ __align__(16) char lds[];
+    const ConvGeom &g = q.g;
+    const int S = tile_stride(g.Ci), nk = g.Kpad / 32;
+    int *tab = reinterpret_cast<int *>(lds + tile_positions(TZ) * S);  // offset of chunk kc, lane group grp
+    const unsigned id = xcd_remap(blockIdx.x, gridDim.x);
+    const int ct = (int)(id % (unsigned)nct), c0 = ct * 16 * NB;
+    int n, z0, y0, x0;
+    tile_origin(q, (int)(id / (unsigned)nct), TZ, n, z0, y0, x0);
+    for (int i = threadIdx.x; i < 4 * nk; i += 256) {
+        const int k = i * 8, tap = k / g.Ci;
+        tab[i] = tap < 27 ? tap_offset(tap, k - tap * g.Ci, S) : 0;
+    }
+    // weights: KC chunks at a time in LDS, in operand order (16 bytes of lane
+    // l of chunk u, block nb at ((u*NB + nb)*64 + l)*16), double buffered
+    char *const wlds = reinterpret_cast<char *>(tab + 4 * ((nk + 3) / 4 * 4));
+    u32x4 wreg[WR];
+    auto weights = [&](int st) {
+#pragma unroll
+        for (int u = 0; u < WR; ++u) {
+            const int i = threadIdx.x + 256 * u, row = i / (KC * 4), kq = st * KC * 4 + i % (KC * 4);
+            wreg[u] = u32x4{0u, 0u, 0u, 0u};
+            if (c0 + row < g.Co && kq < nk * 4)
+                wreg[u] = *reinterpret_cast<const u32x4 *>(wt + (long long)(c0 + row) * g.Kpad + kq * 8);
+        }
+    };
+    auto put = [&](int st) {
+        char *const to = wlds + (st & 1) * (KC * NB * 1024);
+#pragma unroll
+        for (int u = 0; u < WR; ++u) {
+            const int i = threadIdx.x + 256 * u, row = i / (KC * 4), kq = i % (KC * 4);
+            *reinterpret_cast<u32x4 *>(to + (((kq >> 2) * NB + (row >> 4)) * 64 + (kq & 3) * 16 + (row & 15)) * 16) = wreg[u];
+        }
+    };
+    weights(0);
+    tile_stage<TZ, 4>(act, g, n, z0, y0, x0, lds, S);
+    put(0);
+    __syncthreads();
+
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int j = lane & 15, grp = lane >> 4;
+    const char *base[MB];
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+        const int row = w * MB + m;
+        base[m] = lds + ((row / kTy * (kTy + 2) + row % kTy) * (kTx + 2) + j) * S;
+    }
+    f32x4 acc[NB][MB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int m = 0; m < MB; ++m) acc[nb][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // activations of a chunk are fetched while the one before is multiplied
+    auto taps = [&](int kc, bf16x8 (&b)[MB]) {
+        const int off = tab[min(kc, nk - 1) * 4 + grp];
+#pragma unroll
+        for (int m = 0; m < MB; ++m) b[m] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(base[m] + off));
+    };
+    // the last chunk's columns beyond 27*Ci multiply zeros
+    const bool pad = (nk - 1) * 32 + grp * 8 >= 27 * g.Ci;
+    bf16x8 b[2][MB];
+    taps(0, b[0]);
+    const int stages = (nk + KC - 1) / KC;
+    for (int st = 0; st < stages; ++st) {
+        if (st + 1 < stages) weights(st + 1);
+        const char *wl = wlds + (st & 1) * (KC * NB * 1024) + lane * 16;
+        bf16x8 a[2][NB];
+        auto wfetch = [&](int u, bf16x8 (&d)[NB]) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+                d[nb] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(wl + (u * NB + nb) * 1024));
+        };
+        wfetch(0, a[0]);
+#pragma unroll
+        for (int u = 0; u < KC; ++u) {
+            const int kc = st * KC + u;
+            if (kc >= nk) break;
+            if (u + 1 < KC) wfetch(u + 1, a[(u + 1) & 1]);
+            taps(kc + 1, b[(u + 1) & 1]);
+            if (kc == nk - 1 && pad) {
+#pragma unroll
+                for (int m = 0; m < MB; ++m) b[u & 1][m] = zero8();
+            }
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int m = 0; m < MB; ++m)
+                    acc[nb][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u & 1][nb], b[u & 1][m], acc[nb][m], 0, 0, 0);
+        }
+        if (st + 1 < stages) {
+            put(st + 1);
+            __syncthreads();
+        }
+    }
+
+    // lane holds D[co = 4*grp + v][position j] of each (nb, m) block
+    const long long sample = (long long)n * g.D * g.H * g.W;
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+        const int row = w * MB + m, z = z0 + row / kTy, y = y0 + row % kTy, x = x0 + j;
+        if (z >= g.D || y >= g.H || x >= g.W) continue;
+        const long long p = sample + ((long long)z * g.H + y) * g.W + x;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const int cb = c0 + nb * 16 + 4 * grp;
+            if (cb >= g.Co) continue;  // Co is a multiple of 4
+            f32x4 v = acc[nb][m];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (bias) v[e] += bias[cb + e];
+                if (relu) v[e] = v[e] > 0.f ? v[e] : 0.f;
+            }
+            if (out_f) {
+                f32x4 *o = reinterpret_cast<f32x4 *>(out_f + p * g.Co + cb);
+                if (accumulate) {
+                    const f32x4 t = *o;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) (*o)[e] = t[e] + v[e];
+                } else {
+                    *o = v;
+                }
+            }
+            if (out_bf) {
+                *reinterpret_cast<uint2 *>(out_bf + p * g.Co + cb) = make_uint2(pack_bf(v[0], v[1]), pack_bf(v[2], v[3]));
+            }
+        }
+    }
+}
+
 // ---------------------------------------------------------------- weight gradient
 
 // dW[co][k] += sum_p dY[p][co] * X[p + off(tap(k))][ci(k)]
@@ -270,128 +501,155 @@ __global__ __launch_bounds__(256) void k_conv3_wgrad(const bf16_t *__restrict__ 
     }
 }
 
-// ---------------------------------------------------------------- weight gradient, channel-major operands
+// ---------------------------------------------------------------- weight gradient, LDS tiles
 
-// The MFMA operands of the weight gradient run along positions (8
-// consecutive positions of one channel per lane), which channels-last
-// activations hold Ci values apart: the gather above issues one 2-byte load
-// per value.  When rows are a multiple of 8 positions, both operands are
-// first transposed to channel-major [C][P] copies, and then every operand is
-// one 16-byte load: the dY rows directly, the X rows of a tap with dx = -1
-// or +1 from two aligned loads joined by a 16-bit funnel shift (a group of 8
-// positions never crosses a row, so only its first or last value can fall
-// outside the row, and it is zeroed).
+// dW[co][k] += sum_p dY[p][co] * X[p + off(tap)][ci] over tiles of 16 x 4 x
+// TZ positions: a workgroup stages a tile's neighbourhood of X and its dY in
+// LDS (channels last, as they lie in memory) and takes every tap of every
+// channel from there.  The MFMA reduces over 32 positions (two rows of 16), so
+// both operands run along positions, which channels-last data holds Ci apart:
+// ds_read_b64_tr_b16 reads four positions x 16 channels and hands each lane
+// one channel's four positions, and a tap is an address, not a shift.  (The
+// gathering kernel above reads two bytes at a time; channel-major copies of
+// both operands, with a 16-bit funnel shift for dx = -1 and +1 and one load
+// from L2 per operand, took 1407 us for 48 -> 16 channels at 8 x 64^3.)
+//
+// Wave w of WAVES owns the column blocks w, w + WAVES, .. (16 weight columns
+// k each) of 16*NC output channels and keeps their sums in registers over all
+// of its workgroup's tiles; every workgroup writes its partial dW to the
+// workspace, and k_wgrad_reduce adds them up in a fixed order.
+//
+// Bound: LDS reads (two 8-byte reads per lane for each B operand, used for
+// NC MFMAs).  With channel-major copies and now, 8 x 64^3: 48 -> 16 channels
+// 1495 -> 302 us, 16 -> 16 498 -> 121; 8 x 32^3: 96 -> 32 688 -> 249.
+constexpr int kWgWaves = 8;
 
-// [P][C] -> [C][P] (16-bit words) through LDS, 64 positions per workgroup.
-constexpr int kTrMaxC = 128;
-__global__ __launch_bounds__(256) void k_pc_transpose(const bf16_t *__restrict__ src, bf16_t *__restrict__ dst,
-                                                      int P, int C)
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+// 8 consecutive positions of one channel per lane: positions 0..3 of the
+// lane group at `p`, 4..7 at `p + 4*S`; p is the lane's own place for the
+// transposed read (position (lane & 15) / 4, channels 4*(lane & 3) ..)
+__device__ __forceinline__ bf16x8 read_tr(const char *p, int S4)
 {
-    __shared__ bf16_t t[kTrMaxC * 66];
-    const long long p0 = (long long)blockIdx.x * 64;
-    const int np = (int)min(64LL, (long long)P - p0);
-    for (int i = threadIdx.x; i < np * C; i += 256) {
-        const int pp = i / C, c = i - pp * C;
-        t[c * 66 + pp] = src[p0 * C + i];
+    typedef __attribute__((address_space(3))) s16x4 L;
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((L *)(p));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((L *)(p + S4));
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    const s16x8 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    return __builtin_bit_cast(bf16x8, v);
+}
+
+// NBW column blocks per wave (those below nkb exist), NC blocks of 16 output
+// channels from c0 = 16*NC*blockIdx.y
+template <int NC, int NBW, int TZ>
+__global__ __launch_bounds__(64 * kWgWaves) void k_conv3_wgrad_tile(const bf16_t *__restrict__ X,
+                                                                    const bf16_t *__restrict__ dY,
+                                                                    float *__restrict__ part, TileGeom q, int ntiles)
+{
+    extern __shared__ __align__(16) char lds[];
+    const ConvGeom &g = q.g;
+    const int S = tile_stride(g.Ci);
+    constexpr int SY = NC * 32 + (NC == 1 ? 0 : 16);  // dY position stride, bytes
+    char *const ylds = lds + tile_positions(TZ) * S;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int grp = lane >> 4, c0 = 16 * NC * (int)blockIdx.y;
+    const int K = 27 * g.Ci, nkb = (K + 15) / 16;
+    // the lane's place in a transposed read: positions 8*(grp & 1) + (lane & 15)/4
+    // (+4) of row grp/2 of the step's two rows
+    const int xr = 8 * (grp & 1) + ((lane & 15) >> 2);
+    int boff[NBW];  // X: plus the tap and channel of the lane's four columns
+#pragma unroll
+    for (int i = 0; i < NBW; ++i) {
+        const int k = min((w + i * kWgWaves) * 16 + 4 * (lane & 3), K - 4), tap = k / g.Ci;
+        boff[i] = ((grp >> 1) * (kTx + 2) + xr) * S + tap_offset(tap, k - tap * g.Ci, S);
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < 64 * C; i += 256) {
-        const int c = i >> 6, pp = i & 63;
-        if (pp < np) dst[(long long)c * P + p0 + pp] = t[c * 66 + pp];
+    const int aoff = ((grp >> 1) * kTx + xr) * SY + 8 * (lane & 3);
+    f32x4 acc[NBW][NC];
+#pragma unroll
+    for (int i = 0; i < NBW; ++i)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    for (int t = (int)blockIdx.x; t < ntiles; t += (int)gridDim.x) {
+        int n, z0, y0, x0;
+        tile_origin(q, t, TZ, n, z0, y0, x0);
+        tile_stage<TZ, kWgWaves>(X, g, n, z0, y0, x0, lds, S);
+        // dY of the tile: zero outside the sample and beyond Co
+        const long long sample = (long long)n * g.D * g.H * g.W;
+        for (int i = threadIdx.x; i < TZ * kTy * kTx * NC * 4; i += 64 * kWgWaves) {
+            const int c4 = i % (NC * 4), p = i / (NC * 4), px = p % kTx, r = p / kTx;
+            const int x = x0 + px, y = y0 + r % kTy, z = z0 + r / kTy, c = c0 + c4 * 4;
+            uint2 v = make_uint2(0u, 0u);
+            if (x < g.W && y < g.H && z < g.D && c < g.Co)
+                v = *reinterpret_cast<const uint2 *>(dY + (sample + ((long long)z * g.H + y) * g.W + x) * g.Co + c);
+            *reinterpret_cast<uint2 *>(ylds + p * SY + c4 * 8) = v;
+        }
+        __syncthreads();
+        const bool edge = x0 + kTx > g.W || y0 + kTy > g.H || z0 + TZ > g.D;
+#pragma unroll 1
+        for (int r = 0; r < TZ * kTy; r += 2) {
+            const char *yp = ylds + r * kTx * SY + aoff;
+            const char *xp = lds + (r / kTy * (kTy + 2) + r % kTy) * (kTx + 2) * S;
+            bf16x8 a[NC];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) a[c] = read_tr(yp + c * 32, 4 * SY);
+            u32x4 keep = {~0u, ~0u, ~0u, ~0u};
+            if (edge) {
+                // positions outside the sample: X may hold infinities there
+                // that a zero dY would turn into NaN
+                const int rr = r + (grp >> 1);
+                const bool in = y0 + rr % kTy < g.H && z0 + rr / kTy < g.D;
+                const int left = in ? g.W - x0 - 8 * (grp & 1) : 0;  // positions of the lane inside
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    keep[e] = (2 * e < left ? 0xffffu : 0u) | (2 * e + 1 < left ? 0xffff0000u : 0u);
+            }
+#pragma unroll
+            for (int i = 0; i < NBW; ++i) {
+                if (w + i * kWgWaves >= nkb) break;
+                bf16x8 b = read_tr(xp + boff[i], 4 * S);
+                if (edge) b = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, b) & keep);
+#pragma unroll
+                for (int c = 0; c < NC; ++c)
+                    acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[c], b, acc[i][c], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
+    // lane holds D[row co = 4*grp + e][column lane & 15] of each block
+    float *const o = part + (long long)blockIdx.x * g.Co * g.Kpad;
+#pragma unroll
+    for (int i = 0; i < NBW; ++i) {
+        const int k = (w + i * kWgWaves) * 16 + (lane & 15);
+        if (k >= K) continue;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int co = c0 + c * 16 + 4 * grp + e;
+                if (co < g.Co) o[(long long)co * g.Kpad + k] = acc[i][c][e];
+            }
     }
 }
 
-__device__ __forceinline__ u32x4 load8u(const bf16_t *p) { return *reinterpret_cast<const u32x4 *>(p); }
-
-// dW[co][k] += sum_p dYt[co][p] * Xt[ci(k)][p + off(tap(k))]; the same
-// tiling as k_conv3_wgrad (rows = output channels, 16*NB weight columns,
-// 32 positions per MFMA, `pchunk` positions per wave, atomics at the end).
-// Requires W % 8 == 0 and pchunk % 32 == 0.
-template <int NB>
-__global__ __launch_bounds__(256) void k_conv3_wgrad_t(const bf16_t *__restrict__ Xt,
-                                                       const bf16_t *__restrict__ dYt,
-                                                       float *__restrict__ dW, ConvGeom g, int pchunk)
+// dW += the partial sums of all workgroups, in their order; padding columns
+// (k >= 27*Ci) are not touched
+__global__ __launch_bounds__(256) void k_wgrad_reduce(const float *__restrict__ part, float *__restrict__ dW, int n,
+                                                      int K, int Kpad, int parts)
 {
-    const int lane = threadIdx.x & 63;
-    const int j = lane & 15, grp = lane >> 4;
-    const long long wave = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const int K = 27 * g.Ci;
-    const int nkt = (K + 16 * NB - 1) / (16 * NB);
-    const int nct = (g.Co + 15) / 16;
-    const long long nchunks = ((long long)g.P + pchunk - 1) / pchunk;
-    const long long total = nchunks * nkt * nct;
-    if (wave >= total) return;
-    const int kt = (int)(wave % nkt);
-    const long long r2 = wave / nkt;
-    const int ct = (int)(r2 % nct);
-    const int pc = (int)(r2 / nct);
-    const int co = ct * 16 + j;  // A-operand row of this lane
-    const long long HW = (long long)g.H * g.W;
-    const bf16_t *arow = dYt + (long long)min(co, g.Co - 1) * g.P;
-    int kk[NB], dz[NB], dy[NB], dx[NB];
-    const bf16_t *brow[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        kk[nb] = kt * 16 * NB + nb * 16 + j;  // B-operand column of this lane
-        const int kc = kk[nb] < K ? kk[nb] : 0;
-        const int tap = kc / g.Ci;
-        const int ci = kc - tap * g.Ci;
-        dz[nb] = tap / 9 - 1;
-        dy[nb] = (tap / 3) % 3 - 1;
-        dx[nb] = tap % 3 - 1;
-        brow[nb] = Xt + (long long)ci * g.P;
+    __shared__ float red[256];
+    // four lanes' worth of partial sums per weight, 64 weights per workgroup
+    const int e = (int)blockIdx.x * 64 + (threadIdx.x & 63), h = threadIdx.x >> 6;
+    float s = 0.f;
+    if (e < n && e % Kpad < K) {
+        const int lo = parts * h / 4, hi = parts * (h + 1) / 4;
+#pragma unroll 8
+        for (int p = lo; p < hi; ++p) s += part[(long long)p * n + e];
     }
-    f32x4 acc[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int pbeg = pc * pchunk, pend = min(pbeg + pchunk, g.P);
-    const u32x4 zero = {0u, 0u, 0u, 0u};
-    for (int ps = pbeg; ps < pend; ps += 32) {
-        // this lane group's 8 positions: one row segment (W % 8 == 0)
-        const int pf = ps + grp * 8;
-        const bool pin = pf < pend;
-        int n0, z0, y0, x0;
-        decode(g, min(pf, g.P - 8), n0, z0, y0, x0);
-        const u32x4 av = (pin && co < g.Co) ? load8u(arow + pf) : zero;
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            const int zz = z0 + dz[nb], yy = y0 + dy[nb];
-            const bool ok = pin && kk[nb] < K && zz >= 0 && zz < g.D && yy >= 0 && yy < g.H;
-            u32x4 b = zero;
-            if (ok) {
-                const bf16_t *q = brow[nb] + pf + (long long)dz[nb] * HW + (long long)dy[nb] * g.W;
-                const u32x4 v = load8u(q);
-                if (dx[nb] == 0) {
-                    b = v;
-                } else if (dx[nb] < 0) {
-                    // values x0-1 .. x0+6: the last of the group before, then v[0..6]
-                    const unsigned prev = x0 > 0 ? load8u(q - 8)[3] : 0u;
-                    b[0] = __builtin_amdgcn_alignbit(v[0], prev, 16);
-                    b[1] = __builtin_amdgcn_alignbit(v[1], v[0], 16);
-                    b[2] = __builtin_amdgcn_alignbit(v[2], v[1], 16);
-                    b[3] = __builtin_amdgcn_alignbit(v[3], v[2], 16);
-                } else {
-                    // values x0+1 .. x0+8: v[1..7], then the first of the group after
-                    const unsigned next = x0 + 8 < g.W ? load8u(q + 8)[0] : 0u;
-                    b[0] = __builtin_amdgcn_alignbit(v[1], v[0], 16);
-                    b[1] = __builtin_amdgcn_alignbit(v[2], v[1], 16);
-                    b[2] = __builtin_amdgcn_alignbit(v[3], v[2], 16);
-                    b[3] = __builtin_amdgcn_alignbit(next, v[3], 16);
-                }
-            }
-            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av),
-                                                              __builtin_bit_cast(bf16x8, b), acc[nb], 0, 0, 0);
-        }
-    }
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        if (kk[nb] >= K) continue;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int c = ct * 16 + 4 * grp + e;
-            if (c < g.Co) atomicAdd(dW + (long long)c * g.Kpad + kk[nb], acc[nb][e]);
-        }
-    }
+    red[threadIdx.x] = s;
+    __syncthreads();
+    if (h == 0 && e < n && e % Kpad < K)
+        dW[e] += (red[threadIdx.x] + red[threadIdx.x + 64]) + (red[threadIdx.x + 128] + red[threadIdx.x + 192]);
 }
 
 // ---------------------------------------------------------------- small layers
@@ -813,6 +1071,94 @@ static ConvGeom make_conv(int N, int D, int H, int W, int Ci, int Co, int Kpad)
     return g;
 }
 
+// The tiled convolution of a layer (fn null: none).
+struct ConvTilePlan {
+    const void *fn = nullptr;
+    TileGeom q;
+    int nct, blocks, lds;
+};
+
+template <int NB>
+static const void *conv_tile_fn(int mb)
+{
+    return mb == 4 ? reinterpret_cast<const void *>(&k_conv3_tile<NB, 4>)
+                   : reinterpret_cast<const void *>(&k_conv3_tile<NB, 2>);
+}
+
+static ConvTilePlan conv_tile_plan(const ConvGeom &g, const void *out_bf, const void *out_f)
+{
+    ConvTilePlan t;
+    // the kernel stores four channels at once
+    if ((reinterpret_cast<uintptr_t>(out_bf) & 7) || (reinterpret_cast<uintptr_t>(out_f) & 15)) return t;
+    int mb = 4;
+    const int cb = (g.Co + 15) / 16;  // blocks of 16 output channels
+    const int nb = cb <= 4 ? cb : cb % 4 == 0 ? 4 : cb % 3 == 0 ? 3 : 4;
+    const int tab = (g.Kpad / 32 + 3) / 4 * 64 + 2 * conv_chunks(nb) * nb * 1024;
+    t.lds = tile_positions(mb) * tile_stride(g.Ci) + tab;
+    if (mb == 4 && t.lds > 80 * 1024) {
+        mb = 2;
+        t.lds = tile_positions(mb) * tile_stride(g.Ci) + tab;
+    }
+    if (t.lds > kMaxLds) return t;
+    t.nct = (cb + nb - 1) / nb;
+    t.q.g = g;
+    t.q.tx = (g.W + kTx - 1) / kTx;
+    t.q.ty = (g.H + kTy - 1) / kTy;
+    t.q.tz = (g.D + mb - 1) / mb;
+    const long long blocks = (long long)g.N * t.q.tx * t.q.ty * t.q.tz * t.nct;
+    if (blocks >= (1LL << 31)) return t;
+    t.blocks = (int)blocks;
+    t.fn = nb == 4 ? conv_tile_fn<4>(mb) : nb == 3 ? conv_tile_fn<3>(mb) : nb == 2 ? conv_tile_fn<2>(mb) : conv_tile_fn<1>(mb);
+    return t;
+}
+
+// The tiled weight gradient of a layer (fn null: none): parts workgroups per
+// group of 16*NC output channels.
+struct WgradTilePlan {
+    const void *fn = nullptr;
+    TileGeom q;
+    int ntiles, parts, groups, lds;
+};
+
+template <int NC, int TZ>
+static const void *wgrad_tile_fn(int nbw)
+{
+    if (nbw <= 2) return reinterpret_cast<const void *>(&k_conv3_wgrad_tile<NC, 2, TZ>);
+    if (nbw <= 4) return reinterpret_cast<const void *>(&k_conv3_wgrad_tile<NC, 4, TZ>);
+    if (nbw <= 7) return reinterpret_cast<const void *>(&k_conv3_wgrad_tile<NC, 7, TZ>);
+    if (nbw <= 11) return reinterpret_cast<const void *>(&k_conv3_wgrad_tile<NC, 11, TZ>);
+    if (nbw <= 14) return reinterpret_cast<const void *>(&k_conv3_wgrad_tile<NC, 14, TZ>);
+    if (nbw <= 21) return reinterpret_cast<const void *>(&k_conv3_wgrad_tile<NC, 21, TZ>);
+    return nullptr;
+}
+
+static WgradTilePlan wgrad_tile_plan(const ConvGeom &g)
+{
+    WgradTilePlan t;
+    if (g.Co % 4 || g.Co < 4) return t;  // dY is read four channels at a time
+    const int nc = g.Co > 16 ? 2 : 1;
+    const int nbw = ((27 * g.Ci + 15) / 16 + kWgWaves - 1) / kWgWaves;
+    // tiles of 4 planes while two workgroups fit a CU's LDS, else of 2
+    auto lds = [&](int tz) { return tile_positions(tz) * tile_stride(g.Ci) + tz * kTy * kTx * (nc * 32 + (nc == 1 ? 0 : 16)); };
+    const int tz = lds(4) <= 80 * 1024 ? 4 : 2;
+    t.lds = lds(tz);
+    if (t.lds > kMaxLds) return t;
+    t.q.g = g;
+    t.q.tx = (g.W + kTx - 1) / kTx;
+    t.q.ty = (g.H + kTy - 1) / kTy;
+    t.q.tz = (g.D + tz - 1) / tz;
+    const long long tiles = (long long)g.N * t.q.tx * t.q.ty * t.q.tz;
+    if (tiles >= (1LL << 31)) return t;
+    t.ntiles = (int)tiles;
+    t.groups = (g.Co + 16 * nc - 1) / (16 * nc);
+    // two workgroups per CU, and at most 32 MiB of partial sums
+    const long long want = std::min(512LL / t.groups, (32LL << 20) / (4LL * g.Co * g.Kpad));
+    t.parts = (int)std::max(1LL, std::min((long long)t.ntiles, want));
+    if (nc == 1) t.fn = tz == 4 ? wgrad_tile_fn<1, 4>(nbw) : wgrad_tile_fn<1, 2>(nbw);
+    else t.fn = tz == 4 ? wgrad_tile_fn<2, 4>(nbw) : wgrad_tile_fn<2, 2>(nbw);
+    return t;
+}
+
 extern "C" {
 
 int st_nn_kpad(int ci) { return (27 * ci + 31) / 32 * 32; }
@@ -820,17 +1166,25 @@ int st_nn_kpad(int ci) { return (27 * ci + 31) / 32 * 32; }
 st_status st_nn_conv3(const void *act, const void *w, const float *bias, void *out_bf16, float *out_f32,
                       int N, int D, int H, int W, int Ci, int Co, int relu, int accumulate, void *stream)
 {
-    if (Ci % 8 || Co % 4 || Co < 4 || N < 1 || D < 1 || H < 1 || W < 1)
+    if (Ci % 8 || Ci < 8 || Co % 4 || Co < 4 || N < 1 || D < 1 || H < 1 || W < 1)
         return fail(ST_EINVAL, "conv3: Ci must be a multiple of 8 and Co of 4 (got %d, %d)", Ci, Co);
     if ((long long)N * D * H * W >= (1LL << 31)) return fail(ST_EINVAL, "conv3: too many positions");
     const ConvGeom g = make_conv(N, D, H, W, Ci, Co, st_nn_kpad(Ci));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int nb = Co >= 64 ? 4 : (Co >= 32 ? 2 : 1);
-    const long long waves = ((g.P + 63) / 64) * ((Co + 16 * nb - 1) / (16 * nb));
-    const dim3 grid((unsigned)((waves + 3) / 4)), block(256);
     const bf16_t *a = static_cast<const bf16_t *>(act);
     const bf16_t *wt = static_cast<const bf16_t *>(w);
     bf16_t *ob = static_cast<bf16_t *>(out_bf16);
+    const ConvTilePlan t = conv_tile_plan(g, out_bf16, out_f32);
+    if (t.fn) {
+        void *args[] = {&a, &wt, &bias, &ob, &out_f32, const_cast<TileGeom *>(&t.q), const_cast<int *>(&t.nct), &relu,
+                        &accumulate};
+        hipError_t e = hipFuncSetAttribute(t.fn, hipFuncAttributeMaxDynamicSharedMemorySize, t.lds);
+        if (e != hipSuccess) return hip_check(e, "hipFuncSetAttribute(conv3 LDS)");
+        return hip_check(hipLaunchKernel(t.fn, dim3(t.blocks), dim3(256), args, t.lds, s), "conv3 launch");
+    }
+    const int nb = Co >= 64 ? 4 : (Co >= 32 ? 2 : 1);
+    const long long waves = ((g.P + 63) / 64) * ((Co + 16 * nb - 1) / (16 * nb));
+    const dim3 grid((unsigned)((waves + 3) / 4)), block(256);
     if (nb == 4) hipLaunchKernelGGL((k_conv3<4, 4>), grid, block, 0, s, a, wt, bias, ob, out_f32, g, relu, accumulate);
     else if (nb == 2) hipLaunchKernelGGL((k_conv3<2, 4>), grid, block, 0, s, a, wt, bias, ob, out_f32, g, relu, accumulate);
     else hipLaunchKernelGGL((k_conv3<1, 4>), grid, block, 0, s, a, wt, bias, ob, out_f32, g, relu, accumulate);
@@ -840,30 +1194,32 @@ st_status st_nn_conv3(const void *act, const void *w, const float *bias, void *o
 st_status st_nn_conv3_wgrad(const void *x, const void *dy, float *dw, int N, int D, int H, int W, int Ci,
                             int Co, void *stream)
 {
-    if (Ci % 8) return fail(ST_EINVAL, "conv3 wgrad: Ci must be a multiple of 8");
+    if (Ci % 8 || Ci < 8) return fail(ST_EINVAL, "conv3 wgrad: Ci must be a multiple of 8");
     if ((long long)N * D * H * W >= (1LL << 31)) return fail(ST_EINVAL, "conv3 wgrad: too many positions");
     const ConvGeom g = make_conv(N, D, H, W, Ci, Co, st_nn_kpad(Ci));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const bf16_t *xb = static_cast<const bf16_t *>(x), *yb = static_cast<const bf16_t *>(dy);
+    const WgradTilePlan t = wgrad_tile_plan(g);
+    if (t.fn) {
+        void *ws = nullptr;
+        st_status st = workspace_slot(0, (size_t)t.parts * Co * g.Kpad * sizeof(float), s, &ws);
+        if (st != ST_OK) return st;
+        float *part = static_cast<float *>(ws);
+        void *args[] = {&xb, &yb, &part, const_cast<TileGeom *>(&t.q), const_cast<int *>(&t.ntiles)};
+        hipError_t e = hipFuncSetAttribute(t.fn, hipFuncAttributeMaxDynamicSharedMemorySize, t.lds);
+        if (e != hipSuccess) return hip_check(e, "hipFuncSetAttribute(wgrad LDS)");
+        e = hipLaunchKernel(t.fn, dim3(t.parts, t.groups), dim3(64 * kWgWaves), args, t.lds, s);
+        if (e != hipSuccess) return hip_check(e, "conv3 wgrad launch");
+        const int n = Co * g.Kpad;
+        hipLaunchKernelGGL(k_wgrad_reduce, dim3((n + 63) / 64), dim3(256), 0, s, part, dw, n, 27 * Ci, g.Kpad, t.parts);
+        return hip_check(hipGetLastError(), "conv3 wgrad reduce launch");
+    }
     const int pchunk = 2048;
     const int K = 27 * Ci;
     const long long nkt = (K + 63) / 64, nct = (Co + 15) / 16, nch = (g.P + pchunk - 1) / pchunk;
     const long long waves = nkt * nct * nch;
-    hipStream_t s = static_cast<hipStream_t>(stream);
     const dim3 grid((unsigned)((waves + 3) / 4));
-    if (W % 8 == 0 && Ci <= kTrMaxC && Co <= kTrMaxC) {
-        // channel-major copies of both operands in the workspace (slot 0)
-        void *ws = nullptr;
-        st_status st = workspace_slot(0, ((size_t)g.P * Ci + (size_t)g.P * Co) * sizeof(bf16_t), s, &ws);
-        if (st != ST_OK) return st;
-        bf16_t *xt = static_cast<bf16_t *>(ws);
-        bf16_t *dyt = xt + (size_t)g.P * Ci;
-        const dim3 tg((unsigned)((g.P + 63) / 64));
-        hipLaunchKernelGGL(k_pc_transpose, tg, dim3(256), 0, s, static_cast<const bf16_t *>(x), xt, g.P, Ci);
-        hipLaunchKernelGGL(k_pc_transpose, tg, dim3(256), 0, s, static_cast<const bf16_t *>(dy), dyt, g.P, Co);
-        hipLaunchKernelGGL((k_conv3_wgrad_t<4>), grid, dim3(256), 0, s, xt, dyt, dw, g, pchunk);
-        return hip_check(hipGetLastError(), "conv3 wgrad launch");
-    }
-    hipLaunchKernelGGL((k_conv3_wgrad<4>), grid, dim3(256), 0, s, static_cast<const bf16_t *>(x),
-                       static_cast<const bf16_t *>(dy), dw, g, pchunk);
+    hipLaunchKernelGGL((k_conv3_wgrad<4>), grid, dim3(256), 0, s, xb, yb, dw, g, pchunk);
     return hip_check(hipGetLastError(), "conv3 wgrad launch");
 }
 
