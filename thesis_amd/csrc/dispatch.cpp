@@ -243,8 +243,12 @@ static st_status resolve(const st_params *p, Cfg &c, bool mixed)
             c.variant = ST_V_BASE;
             c.cx = 1;
         } else {
-            const bool march_ok = (c.dtype == ST_F32 && c.r <= 8) ||
-                                  (c.dtype == ST_F64 && (c.r == 1 || c.r == 2 || c.r == 4));
+            // FP32 up to radius 14, FP64 up to 8 in 3D (us per sweep, plain /
+            // this: FP32 320x256x256 R=14 602 / 311, R=16 394 / 1206; FP64
+            // 192^3 R=3 86 / 25, R=8 125 / 110, R=12 189 / 227)
+            const bool march_ok = c.dims == 3 ? c.r <= (c.dtype == ST_F64 ? 8 : 14)
+                                              : (c.dtype == ST_F32 && c.r <= 8) ||
+                                                    (c.dtype == ST_F64 && (c.r == 1 || c.r == 2 || c.r == 4));
             c.variant = march_ok ? ST_V_SMEM_REGISTER : ST_V_BASE;
             if (!march_ok) c.cx = 1;
         }
@@ -391,7 +395,7 @@ st_status stencil_dispatch(const st_params *p, void *d_u1, void *d_u2, void *str
         } else {
             // the row form stores whole rows when both shells are equal
             // (a shell cell then holds the same bits at every sweep)
-            if (c.variant == ST_V_SMEM_REGISTER && c.kind == 4 && c.iters > 1)
+            if (c.variant == ST_V_SMEM_REGISTER && (c.kind == 4 || c.kind == 8) && c.iters > 1)
                 s = rows_shell_check(c, d_u1, d_u2, hs, &c.shell_eq);
             void *a = d_u1, *b = d_u2;
             for (int i = 0; i < c.iters && s == ST_OK; ++i) {

@@ -72,6 +72,12 @@ st_status resolve_rows(Cfg &c);
 st_status resolve_rows_coop(Cfg &c);
 st_status run_rows_coop(const Cfg &c, void *u1, void *u2, hipStream_t s, int *in_u2);
 st_status launch_rows(const Cfg &c, const void *in, void *out, hipStream_t s);
+bool rows_consecutive(const Cfg &c);  // the row form would take its consecutive layout
+// SMEM_REGISTER tile form, one sweep (sweep_tile.hip); eligible: the
+// library's choice for the shape.
+bool tile_eligible(const Cfg &c);
+st_status resolve_tile(Cfg &c);
+st_status launch_tile(const Cfg &c, const void *in, void *out, hipStream_t s);
 // 16-bit storage modes on the geometry of `c` (FP32 arithmetic, JACOBI
 // weight c.weight): defect d = round16(w*sum(x) - x), else the correction
 // e' = round16(widen(d) + w*sum(widen(e))); the output's shell must be zero

@@ -130,10 +130,15 @@ static const MarchEntry *best_march(int d, int f64, int r, int cx, int ty)
 st_status resolve_march(Cfg &c)
 {
     // form: 1 register march, 2 row streaming; the library's choice is the
-    // row-streaming form wherever it applies (3D, radius 1..4: 599 vs 582
-    // GCells/s at 512^3 R=1, 2.9x at 384^3 R=4), the march elsewhere
+    // tile form where it is ahead (sweep_tile.hip), else the row-streaming
+    // form wherever it applies (3D, radius 1..4: 599 vs 582 GCells/s at 512^3
+    // R=1, 2.9x at 384^3 R=4), the march elsewhere
     {
         const bool heur0 = c.heuristic || c.bx <= 0;
+        if (c.form == 0 && heur0 && tile_eligible(c)) {
+            c.heuristic = 1;
+            return resolve_tile(c);
+        }
         if (c.form == 2 || (c.form == 0 && heur0 && rows_eligible(c))) {
             if (heur0) c.heuristic = 1;
             return resolve_rows(c);
@@ -196,6 +201,7 @@ st_status resolve_march(Cfg &c)
 st_status launch_march(const Cfg &c, const void *in, void *out, hipStream_t s)
 {
     if (c.kind == 4) return launch_rows(c, in, out, s);
+    if (c.kind == 8) return launch_tile(c, in, out, s);
     const MarchEntry *e = find_march(c.dims, c.dtype == ST_F64, c.r, c.cx, c.cy);
     if (!e) return fail(ST_EUNSUPPORTED, "no SMEM_REGISTER kernel for r=%d cx=%d ty=%d", c.r, c.cx, c.cy);
     const int es = c.dtype == ST_F64 ? 8 : 4;

@@ -980,6 +980,13 @@ static const void *rowc_fn_mode(const Cfg &c, int cx, int mode, bool f16, int *t
     return rowc_fn_d<float, RM_SWEEP, false>(c.op, c.r, cx, threads);
 }
 
+bool rows_consecutive(const Cfg &c)
+{
+    const int cx = c.dims == 3 ? rowc_cx(c) : 0;
+    int threads = 0;
+    return cx && rowc_fn_mode(c, cx, RM_SWEEP, false, &threads) && threads / 64 >= 2 * c.r;
+}
+
 // The row kernel a resolved configuration launches.
 static const void *rows_kernel(const Cfg &c, int mode, bool f16, int *threads)
 {

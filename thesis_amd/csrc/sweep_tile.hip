@@ -1,0 +1,379 @@
+// SMEM_REGISTER family, tile form: one sweep, any row width and alignment,
+// FP32 up to radius 12 and FP64 up to radius 6 (3D).
+//
+// The reference's smem_register kernels keep an xy tile in shared memory and
+// each thread's z column in registers (src/stencil_kernel_smem_register.cu,
+// src/prefetch_smem.cu:151-258).  Here a workgroup of 8 waves owns a tile of
+// 64 columns x 32*RY rows and marches it along z over a chunk of planes:
+//   * per plane, the tile and its halo (R rows above and below, R columns
+//     rounded up to whole quads left and right) go from registers, where the
+//     plane was prefetched, to one of two LDS planes; one barrier per plane.
+//     The loads are raw buffer loads: what lies outside the field reads 0,
+//     what lies past a row's end reads the next row, and neither is ever
+//     used by an interior cell, so no width or alignment is special;
+//   * a lane owns a quad of 4 consecutive columns in RY adjacent rows (16
+//     lanes along x, 4 along y): x neighbours come from the quads beside its
+//     own, y neighbours from the same quad of the rows around it, which the
+//     RY rows share;
+//   * z: a ring of the R previous planes and R running partial sums per cell,
+//     as in the row form (sweep_rows.hip): plane m starts P_m with its x, y
+//     and z-previous terms in the reference's order and is added to P_{m-1} ..
+//     P_{m-R}, the last of which it completes.
+// The halo a tile loads is (64+2R)(32*RY+2R) cells for 64*32*RY; the row form
+// reads 1 + 2R/rows rows per row, up to 2.3 where registers leave it few
+// rows, and the register march 2R + rows (sweep_march.hip).
+//
+// Bound: VALU and the LDS reads for wide stars (512^3 R = 8: 188 us of VALU,
+// 173 of the field's bytes at 6.2 TB/s; measured 286), memory for narrow ones.
+// Before (row form, register march or plain kernel, whichever was faster) and
+// now, us per sweep: FP32 333x251x207 R = 2 49 -> 24, R = 4 147 -> 34; 512^3
+// R = 6 603 -> 231, R = 8 906 -> 286, R = 12 1151 -> 411; FP64 384^3 R = 4
+// 263 -> 205, R = 3 825 -> 173 (of these, whole FP64 quads in LDS with their
+// two-way bank conflicts: R = 4 428).
+#include <algorithm>
+#include <utility>
+
+#include "st_device.hpp"
+#include "st_internal.hpp"
+
+namespace st {
+
+constexpr int kTileX = 64, kTileWaves = 8;
+
+struct TileArgs {
+    int nx, ny, nz;
+    long long sz;            // nx*ny
+    int tx, ty, zchunk, ntiles;
+    const int *eq;           // 1 when both buffers' shells are equal (whole
+                             // rows are stored then, shell cells unchanged)
+};
+
+// columns of halo on each side: the radius rounded up to whole quads
+__host__ __device__ constexpr int tile_ra(int r) { return (r + 3) / 4 * 4; }
+
+// 16-byte words per row, rows and words per thread of a staged plane
+template <int R, int RY, typename T> constexpr int tile_row_words() { return (kTileX + 2 * tile_ra(R)) * (int)sizeof(T) / 16; }
+template <int R, int RY> constexpr int tile_rows() { return 32 * RY + 2 * R; }
+template <int R, int RY, typename T> constexpr int tile_words()
+{
+    return (tile_row_words<R, RY, T>() * tile_rows<R, RY>() + 64 * kTileWaves - 1) / (64 * kTileWaves);
+}
+template <int R, int RY, typename T> constexpr int tile_lds() { return 2 * tile_rows<R, RY>() * tile_row_words<R, RY, T>() * 16; }
+
+// f(0), f(1), .. with constant arguments, until one returns false (a plain
+// unrolled loop of this size exceeds the unroller's limit from radius 9)
+template <int... I, typename F>
+__device__ __forceinline__ void each_phase(std::integer_sequence<int, I...>, F f)
+{
+    (void)(f(std::integral_constant<int, I>{}) && ...);
+}
+
+template <int OP, int R, int RY, typename T>
+__global__ __launch_bounds__(64 * kTileWaves) void k_tile(const T *__restrict__ in, T *__restrict__ out, TileArgs a, T kc)
+{
+    constexpr int RA = tile_ra(R), RW = tile_row_words<R, RY, T>(), ROWS = tile_rows<R, RY>(), NW = tile_words<R, RY, T>();
+    constexpr int ES = (int)sizeof(T);
+    constexpr int QN = RA / 4;                            // quads of x halo per side
+    typedef unsigned int W4 __attribute__((ext_vector_type(4)));
+    // many registers of state: keep the LDS reads near their use
+    constexpr bool tight = 2 * R * RY * ES > 96;
+    extern __shared__ __align__(16) W4 lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const unsigned id = xcd_remap(blockIdx.x, gridDim.x);
+    const int tx = (int)(id % (unsigned)a.tx), ty = (int)(id / (unsigned)a.tx % (unsigned)a.ty),
+              tz = (int)(id / (unsigned)(a.tx * a.ty));
+    const int x0 = tx * kTileX, y0 = ty * 32 * RY;
+    const int z0 = tz * a.zchunk, z1 = min(z0 + a.zchunk, a.nz);
+    const int k_lo = max(z0, R), k_hi = min(z1, a.nz - R);
+    if (k_lo >= k_hi) return;
+    const bool eqs = a.eq != nullptr && *a.eq != 0;
+
+    // staging: word i of the plane is at row i / RW, 16-byte word i % RW
+    unsigned go[NW];
+    int to[NW];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+        const int q = tid + i * 64 * kTileWaves, r = q / RW, c = q - r * RW;
+        to[i] = ES == 4 ? q : r * RW + (c & 1) * (RW / 2) + (c >> 1);
+        // rows above and columns left of the field: negative offsets, out of
+        // the buffer's range (words past the plane's last row: likewise)
+        go[i] = r < ROWS ? (unsigned)(((y0 - R + r) * a.nx + x0 - RA) * ES + c * 16) : 0x80000000u;
+    }
+    W4 pf[NW];
+    const long long plane = a.sz * ES;
+    auto load_plane = [&](int k) {
+        k = min(max(k, 0), a.nz - 1);
+        const char *p = reinterpret_cast<const char *>(in) + k * plane;
+        const long long left = (a.nz - k) * plane;
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<char *>(p), 0, (int)min(left, 0x7fffffffLL), 0x00020000);
+#pragma unroll
+        for (int i = 0; i < NW; ++i) pf[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)go[i], 0, 0);
+    };
+
+    // the lane's cells: quad at column x, rows y .. y + RY - 1
+    const int qx = lane & 15, x = x0 + 4 * qx, ry = (w * 4 + (lane >> 4)) * RY, y = y0 + ry;
+    const bool whole = x >= R && x + 4 <= a.nx - R, inrow = x < a.nx;
+    const unsigned so = (unsigned)((y * a.nx + x) * ES);
+    // LDS word of the lane's quad QN quads to the left, in the row R above y
+    const int lw = ry * RW + qx;
+
+    T ring[R][RY][4], part[R][RY][4];
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int r = 0; r < RY; ++r)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) ring[i][r][c] = part[i][r][c] = (T)0;
+
+    // An FP64 quad is kept as two 16-byte halves half a row apart, so that the
+    // 16 lanes of a read are contiguous (whole 32-byte quads: two-way bank
+    // conflicts).
+    constexpr int QS = ES == 4 ? 1 : RW / 2;  // words from half to half
+    auto quad = [&](const W4 *p, T (&v)[4]) {
+        if constexpr (ES == 4) {
+            const W4 q = *p;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] = __uint_as_float(q[c]);
+        } else {
+            typedef double D2 __attribute__((ext_vector_type(2)));
+            const D2 q0 = __builtin_bit_cast(D2, p[0]), q1 = __builtin_bit_cast(D2, p[QS]);
+            v[0] = q0[0]; v[1] = q0[1]; v[2] = q1[0]; v[3] = q1[1];
+        }
+    };
+
+    const int m_lo = k_lo - R, m_hi = k_hi + R;
+    load_plane(m_lo);
+    // planes in phases of R, unrolled, so that the ring and the partial sums
+    // rotate through their slots with no register moves
+    for (int m0 = m_lo; m0 < m_hi; m0 += R) {
+        each_phase(std::make_integer_sequence<int, R>{}, [&](auto phase) {
+            constexpr int rp = decltype(phase)::value;
+            const int m = m0 + rp;
+            if (m >= m_hi) return false;
+            __builtin_amdgcn_sched_barrier(0);
+            W4 *const buf = lds + ((m - m_lo) & 1) * (ROWS * RW);
+#pragma unroll
+            for (int i = 0; i < NW; ++i) {
+                if ((i + 1) * 64 * kTileWaves <= ROWS * RW || tid + i * 64 * kTileWaves < ROWS * RW) buf[to[i]] = pf[i];
+            }
+            if (m + 1 < m_hi) load_plane(m + 1);
+            __syncthreads();
+            const W4 *const at = buf + lw;
+            T s[RY][4], cur[RY][4];
+            // x terms: own quad and the QN quads on each side
+#pragma unroll
+            for (int r = 0; r < RY; ++r) {
+                T v[4 * (2 * QN + 1)];
+#pragma unroll
+                for (int q = 0; q < 2 * QN + 1; ++q) {
+                    T t[4];
+                    quad(at + (R + r) * RW + q, t);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) v[4 * q + c] = t[c];
+                }
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    cur[r][c] = v[RA + c];
+                    T u = v[RA + c - R];
+#pragma unroll
+                    for (int d = R - 1; d >= 1; --d) u += v[RA + c - d];
+#pragma unroll
+                    for (int d = 1; d <= R; ++d) u += v[RA + c + d];
+                    s[r][c] = u;
+                }
+                if constexpr (tight) __builtin_amdgcn_sched_barrier(0);
+            }
+            // y terms: rows y-R .. y+RY-1+R in order, each for the rows it neighbours
+#pragma unroll
+            for (int t = -R; t < RY + R; ++t) {
+                T v[4];
+                if (t >= 0 && t < RY) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) v[c] = cur[t][c];
+                } else {
+                    quad(at + (R + t) * RW + QN, v);
+                }
+#pragma unroll
+                for (int r = 0; r < RY; ++r)
+                    if (t != r && t - r >= -R && t - r <= R)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) s[r][c] += v[c];
+                if constexpr (tight)
+                    if ((t + R) % 3 == 2) __builtin_amdgcn_sched_barrier(0);
+            }
+            // z-previous terms: logical ring[i] = plane m-R+i, in slot (rp+i) % R;
+            // plane m is the next z-next term of P_{m-R} .. P_{m-1}
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+#pragma unroll
+                for (int r = 0; r < RY; ++r)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        s[r][c] += ring[(rp + i) % R][r][c];
+                        part[(rp + i) % R][r][c] += cur[r][c];
+                    }
+            // P_{m-R} (slot rp) is complete
+            const int k = m - R;
+            if (k >= k_lo) {
+                char *const po = reinterpret_cast<char *>(out) + k * plane;
+#pragma unroll
+                for (int r = 0; r < RY; ++r) {
+                    T res[4];
+                    finish_sums<OP>(part[rp][r], ring[rp][r], kc, res);
+                    if (!interior1(y + r, a.ny, R) || !inrow) continue;
+                    T *const p = reinterpret_cast<T *>(po + (so + (unsigned)(r * a.nx * ES)));
+                    if (whole || (eqs && x + 4 <= a.nx)) {
+                        typedef T V4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+                        V4 v;
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            const T mine = res[c], held = ring[rp][r][c];
+                            v[c] = whole || interior1(x + c, a.nx, R) ? mine : held;
+                        }
+                        *reinterpret_cast<V4 *>(p) = v;
+                    } else {
+#pragma unroll
+                        for (int c = 0; c < 4; ++c)
+                            if (x + c >= R && x + c < a.nx - R) p[c] = res[c];
+                    }
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < RY; ++r)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    ring[rp][r][c] = cur[r][c];
+                    part[rp][r][c] = s[r][c];
+                }
+            return true;
+        });
+    }
+}
+
+// ---------------------------------------------------------------- host side
+
+struct TileKernel {
+    const void *fn = nullptr;
+    int lds = 0, words = 0;  // LDS bytes; 32-bit words of ring and partial sums per lane
+};
+
+template <int R, int RY, typename T>
+static TileKernel tile_kernel(int op)
+{
+    constexpr int words = 2 * R * RY * 4 * (int)sizeof(T) / 4;
+    // built where the kernel leaves no or few spills
+    if constexpr (words > (RY == 2 ? 112 : 96)) return {};
+    else
+        return {op == OP_THESIS ? reinterpret_cast<const void *>(&k_tile<OP_THESIS, R, RY, T>)
+                                : reinterpret_cast<const void *>(&k_tile<OP_JACOBI, R, RY, T>),
+                tile_lds<R, RY, T>(), words};
+}
+
+template <int RY, typename T>
+static TileKernel tile_kernel_r(int op, int r)
+{
+    switch (r) {
+#define TK(R) case R: return tile_kernel<R, RY, T>(op);
+    TK(1) TK(2) TK(3) TK(4) TK(5) TK(6) TK(7) TK(8)
+    TK(9) TK(10) TK(11) TK(12) TK(13) TK(14) TK(15) TK(16)
+#undef TK
+    default: return {};
+    }
+}
+
+static TileKernel tile_kernel_for(const Cfg &c, int ry)
+{
+    if (c.dtype == ST_F64) return ry == 2 ? tile_kernel_r<2, double>(c.op, c.r) : tile_kernel_r<1, double>(c.op, c.r);
+    return ry == 2 ? tile_kernel_r<2, float>(c.op, c.r) : tile_kernel_r<1, float>(c.op, c.r);
+}
+
+// The library's choice among the SMEM_REGISTER forms (us per sweep, the
+// other forms' best / this one):
+//   * below 2^20 cells the plain kernel is AUTO's choice and the other forms
+//     stay as they were; from radius 6 the few tiles of a small grid march
+//     2R planes each for a short chunk, so the line lies at 2^22 cells (FP32
+//     R = 8 128^3 20 / 27, 192^3 61 / 36; R = 5 128^3 24 / 22);
+//   * rows of 256, 384 or 512 columns stay with the consecutive row layout,
+//     which reads every row once per 8 to 16 rows and is level or ahead
+//     (384^3 FP32 R = 4 92 / 100, 512^3 R = 2 203 / 218, 256^3 R = 4 29 / 29;
+//     FP64 256^3 R = 4 50 / 53);
+//   * rows over 512 columns of small 16-byte stars stay with the quad row
+//     layout (640x320x200 FP32 R = 1 67 / 70, FP64 R = 2 121 / 140);
+//   * else the tile is ahead: 320^3 FP32 R = 2 59 / 54, R = 4 75 / 61; widths
+//     that are no multiple of 4, which only the register march took, 1.25x
+//     (R = 1) to 4.3x (R = 4).
+bool tile_eligible(const Cfg &c)
+{
+    if (c.dims != 3 || (c.dtype != ST_F32 && c.dtype != ST_F64)) return false;
+    const long long cells = (long long)c.nx * c.ny * c.nz, es = c.dtype == ST_F64 ? 8 : 4;
+    if (cells <= (1LL << 20) || (c.r >= 6 && cells < (1LL << 22))) return false;
+    // 32-bit byte offsets within a plane and its halo
+    if (((long long)c.nx * (c.ny + 2 * c.r + 64) + 128) * es >= (1LL << 30)) return false;
+    if (c.r <= 4 && c.nx % 4 == 0 && (rows_consecutive(c) || (c.nx > 512 && c.r <= (es == 8 ? 2 : 1))))
+        return false;
+    return tile_kernel_for(c, 1).fn != nullptr;
+}
+
+st_status resolve_tile(Cfg &c)
+{
+    int dev = 0, cus = 256;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+        cus = 256;
+    // rows per lane and z chunk of the least busiest-CU work: rounds of
+    // workgroups x planes marched x rows per lane (a plane costs a fixed part
+    // beside its rows, hence the + 0.5)
+    double best = -1;
+    for (int ry = 1; ry <= 2; ++ry) {
+        const TileKernel t = tile_kernel_for(c, ry);
+        if (!t.fn) continue;
+        const int per_cu = t.words <= 40 && t.lds <= kMaxLds / 2 ? 2 : 1;
+        const long long xy = (long long)((c.nx + kTileX - 1) / kTileX) * ((c.ny + 32 * ry - 1) / (32 * ry));
+        for (int nch = 1; nch <= c.nz; ++nch) {
+            const int ch = (c.nz + nch - 1) / nch;
+            if (nch > 1 && ch < 3) break;
+            const long long n = xy * ((c.nz + ch - 1) / ch);
+            const double cost = (double)((n + cus * per_cu - 1) / (cus * per_cu)) * (ch + 2 * c.r) * (ry + 0.6) * (per_cu == 2 ? 1.6 : 1.0);
+            if (best < 0 || cost < best) {
+                best = cost;
+                c.cy = ry;
+                c.zchunk = ch;
+                c.lds = t.lds;
+                c.gx = (int)n;
+            }
+        }
+    }
+    if (best < 0) return fail(ST_EUNSUPPORTED, "tile form: no kernel for radius %d", c.r);
+    c.kind = 8;
+    c.cx = 4;
+    c.bx = kTileX;
+    c.by = 32 * c.cy;
+    c.bz = c.zchunk;
+    c.gy = c.gz = 1;
+    c.tsteps = 1;
+    return ST_OK;
+}
+
+st_status launch_tile(const Cfg &c, const void *in, void *out, hipStream_t s)
+{
+    const TileKernel t = tile_kernel_for(c, c.cy);
+    if (!t.fn) return fail(ST_EUNSUPPORTED, "tile form: no kernel for radius %d", c.r);
+    TileArgs a;
+    a.nx = c.nx; a.ny = c.ny; a.nz = c.nz;
+    a.sz = (long long)c.nx * c.ny;
+    a.tx = (c.nx + kTileX - 1) / kTileX;
+    a.ty = (c.ny + 32 * c.cy - 1) / (32 * c.cy);
+    a.zchunk = c.zchunk;
+    a.ntiles = c.gx;
+    a.eq = c.shell_eq;
+    double kd = c.op == OP_THESIS ? (double)(2 * c.dims * c.r) : c.weight;
+    float kf = (float)kd;
+    void *args[] = {&in, &out, &a, c.dtype == ST_F64 ? static_cast<void *>(&kd) : static_cast<void *>(&kf)};
+    hipError_t e = hipFuncSetAttribute(t.fn, hipFuncAttributeMaxDynamicSharedMemorySize, t.lds);
+    if (e != hipSuccess) return hip_check(e, "hipFuncSetAttribute(tile LDS)");
+    return hip_check(hipLaunchKernel(t.fn, dim3(c.gx), dim3(64 * kTileWaves), args, t.lds, s), "tile launch");
+}
+
+}  // namespace st
