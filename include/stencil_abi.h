@@ -205,7 +205,8 @@ st_status stencil_sweep(const st_params *p, const void *d_in, void *d_out, void 
  * reference it is d_u1 for an even iteration count.  The COOP variant
  * schedules its fused passes so that the result lands in the same buffer as
  * the per-sweep variants; the interior of the other buffer then holds an
- * intermediate state, not sweep iterations-1.  If elapsed_ms is not NULL the
+ * intermediate state, not sweep iterations-1 (AUTO: as the family that
+ * stencil_launch_config names).  If elapsed_ms is not NULL the
  * call brackets the sweep loop with HIP events on `stream`, waits for the
  * stop event and stores the time in milliseconds (host set-up excluded). */
 st_status stencil_dispatch(const st_params *p, void *d_u1, void *d_u2, void *stream,

@@ -72,3 +72,27 @@ def test_block_form_quotient_at_the_limits(gpu, oracle, dt, scale):
     (g1, g2), _ = _run(st, p, u, np.zeros_like(u))
     _same(g1, a)
     _same(g2, b)
+
+
+@pytest.mark.parametrize("op", [0, 1])
+@pytest.mark.parametrize("its", [8, 9, 24])
+def test_block_form_without_last_single_pass(gpu, oracle, op, its):
+    """Planes whose family is the streaming form: the result, and the shell
+    of the other buffer, whose interior is then unspecified."""
+    st = gpu
+    nx, ny = 2056, 2049
+    print("[case] block, no single pass", op, its, flush=True)
+    rng = np.random.default_rng(its)
+    u1, u2 = (rng.random((1, ny, nx)).astype(np.float32) for _ in range(2))
+    p = st.StencilParams.make(nx=nx, ny=ny, nz=1, dimensions=2, radius=1, iterations=its, op=op, variant="auto",
+                              heuristic=1)
+    cfg = st.launch_config(p)
+    assert cfg["temporal_steps"] in (5, 7, 9) and cfg["launches"] * cfg["temporal_steps"] < its + 2 * cfg["temporal_steps"]
+    a, b = u1.copy().reshape(ny, nx), u2.copy().reshape(ny, nx)
+    oracle.run(a, b, 2, 1, op, its)
+    got, in_u2 = _run(st, p, u1, u2)
+    assert in_u2 == bool(its % 2)
+    _same(got[its % 2].reshape(ny, nx), (a, b)[its % 2])
+    other, want = got[1 - its % 2].reshape(ny, nx), (a, b)[1 - its % 2]
+    for cut in (np.s_[0], np.s_[-1], np.s_[:, 0], np.s_[:, -1]):
+        _same(other[cut], want[cut])

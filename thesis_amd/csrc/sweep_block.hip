@@ -15,15 +15,18 @@
 // whose shell levels 0, 2, 4, .. see and the buffer it writes (`out`) the
 // one of levels 1, 3, ..: the shell's two values are loaded once and change
 // places at every level, and equal and different shells are one path with
-// no comparison beforehand.  The last pass is a single sweep, so both
-// buffers end as single sweeps leave them.
+// no comparison beforehand.  Where AUTO would name a per-sweep family the
+// last pass is a single sweep, so both buffers end as single sweeps leave
+// them; where it would name the streaming form, which leaves an earlier state
+// in the other buffer, there is no such pass (24 sweeps of 8192^2 FP32
+// JACOBI: streaming form 603 us, with it 695, without it 521).
 //
 // Bound: launches up to 512^2 (a launch per sweep costs 2.5 us, a pass of 9
 // sweeps about 7), above that the VALU: a block computes every row at every
 // level, 64*32 cells for (64-2*steps)*(32-2*steps) stored.  64 sweeps, FP32
 // JACOBI, before (plain kernel below 2048^2, streaming form above) and now:
 // 256^2 172 -> 61 us, 1024^2 322 -> 100, 2048^2 452 -> 178, 4096^2 696 ->
-// 408, 16384^2 6.04 -> 5.45 ms; different shells, which the streaming form
+// 408, 16384^2 6.00 -> 5.26 ms; different shells, which the streaming form
 // sweeps singly, 4096^2 THESIS 1946 -> 552 us.
 #include <algorithm>
 
@@ -138,19 +141,19 @@ static int blocks_along(int n, int len, int steps)
     return n <= len ? 1 : (n - len + stride - 1) / stride + 1;
 }
 
-// Passes of a dispatch of `iters` sweeps: `n` passes of an odd number of
-// sweeps each, at most `most`, then one single sweep; n + 1 has the parity
-// of iters.  Pass i has 1 + 2*(q + (i < rem)) sweeps.
+// Passes of a dispatch: `n` passes of an odd number of sweeps each, at most
+// c.block_steps, then `single` sweeps (0 or 1); their number has the parity
+// of the sweeps'.  Pass i has 1 + 2*(q + (i < rem)) sweeps.
 struct BlockPlan {
-    int n, q, rem;
+    int n, q, rem, single;
 };
-static BlockPlan block_plan(int iters, int most)
+static BlockPlan block_plan(const Cfg &c)
 {
-    const int m = iters - 1;  // sweeps before the last single one
-    int n = (m + most - 1) / most;
-    if ((n ^ m) & 1) ++n;     // n odd numbers sum to m
+    const int single = c.variant == ST_V_COOP ? 0 : 1, m = c.iters - single;
+    int n = (m + c.block_steps - 1) / c.block_steps;
+    if ((n ^ m) & 1) ++n;  // n odd numbers sum to m
     const int pairs = (m - n) / 2;
-    return {n, n ? pairs / n : 0, n ? pairs % n : 0};
+    return {n, n ? pairs / n : 0, n ? pairs % n : 0, single};
 }
 
 static BlockArgs block_args(const Cfg &c, int steps)
@@ -171,7 +174,8 @@ static BlockArgs block_args(const Cfg &c, int steps)
 // blocks are at most two waves per SIMD the launches decide (9); above that
 // 7, and 5 for THESIS, whose quotient makes the halo dearer (4096^2 634 / 552
 // / 605 / 751).  Planes of 2^29 cells and more stay with the streaming form,
-// which is level there with equal shells (32768^2 23.6 against 22.1 ms).
+// which is level there with equal shells (32768^2 23.6 against 22.1 ms;
+// 16384^2 24 sweeps 2.03 against 2.10 here, 64 sweeps 6.00 against 5.26).
 void resolve_block(Cfg &c)
 {
     c.block_steps = 0;
@@ -184,7 +188,11 @@ void resolve_block(Cfg &c)
     c.block_steps = waves(9) <= 2048 ? 9 : (c.op == OP_THESIS && waves(7) > 8192 ? 5 : 7);
 }
 
-int block_launches(const Cfg &c) { return block_plan(c.iters, c.block_steps).n + 1; }
+int block_launches(const Cfg &c)
+{
+    const BlockPlan p = block_plan(c);
+    return p.n + p.single;
+}
 
 template <int OP, typename T>
 static hipError_t block_launch(const void *in, void *out, const BlockArgs &a, double kc, hipStream_t s)
@@ -196,12 +204,12 @@ static hipError_t block_launch(const void *in, void *out, const BlockArgs &a, do
 
 st_status run_block(const Cfg &c, void *u1, void *u2, hipStream_t s, int *in_u2)
 {
-    const BlockPlan p = block_plan(c.iters, c.block_steps);
+    const BlockPlan p = block_plan(c);
     const double kc = c.op == OP_THESIS ? (double)(2 * c.dims) : c.weight;
     auto launch = c.dtype == ST_F64 ? (c.op == OP_THESIS ? &block_launch<OP_THESIS, double> : &block_launch<OP_JACOBI, double>)
                                     : (c.op == OP_THESIS ? &block_launch<OP_THESIS, float> : &block_launch<OP_JACOBI, float>);
     *in_u2 = c.iters & 1;
-    for (int i = 0; i <= p.n; ++i) {
+    for (int i = 0; i < p.n + p.single; ++i) {
         const hipError_t e = launch(u1, u2, block_args(c, i < p.n ? 1 + 2 * (p.q + (i < p.rem)) : 1), kc, s);
         if (e != hipSuccess) return hip_check(e, "block launch");
         std::swap(u1, u2);
