@@ -71,6 +71,23 @@ __device__ __forceinline__ void finish_sums(const T (&sum)[N], const T (&centre)
     }
 }
 
+// finish() of one sum whose chain starts with 0 (never -0), the THESIS
+// quotient as above: `odd` is set where finish() itself has to be taken.
+// A sweep of THESIS, division / this: 256^3 R = 1 23.1 / 19.9 us, 512^3 R = 1
+// 145 / 101, 384^3 R = 4 112 / 104.
+template <int OP, typename T>
+__device__ __forceinline__ T finish_fast(T sum, T centre, T kc, bool &odd)
+{
+    if constexpr (OP == OP_THESIS) {
+        const T rk = (T)1 / kc;
+        const T q = sum * rk;
+        odd |= __builtin_isfpclass(q, 0x0003 | 0x0204 | 0x0090);  // NaN, +-infinity, +-subnormal
+        return __builtin_elementwise_fma(__builtin_elementwise_fma(-kc, q, sum), rk, q) - centre;
+    } else {
+        return finish<OP>(sum, centre, kc);
+    }
+}
+
 __device__ __forceinline__ bool interior1(int i, int n, int r) { return i >= r && i < n - r; }
 
 // Cross-lane read of a 32-bit or 64-bit value from lane `src` (0..63; any

@@ -433,8 +433,13 @@ __global__ __launch_bounds__((rows_max_threads<R, CX, T, MODE, HS>())) void k_ro
             if (out_plane) {
                 if constexpr (MODE == RM_SWEEP) {
                     T res[CX];
+                    bool odd = false;
 #pragma unroll
-                    for (int c = 0; c < CX; ++c) res[c] = finish<OP>(part[rp][c], ring[rp][c], kc);
+                    for (int c = 0; c < CX; ++c) res[c] = finish_fast<OP>(part[rp][c], ring[rp][c], kc, odd);
+                    if (OP == OP_THESIS && __builtin_expect(__any(odd), 0)) {
+#pragma unroll
+                        for (int c = 0; c < CX; ++c) res[c] = finish<OP>(part[rp][c], ring[rp][c], kc);
+                    }
                     T *row = static_cast<T *>(out_) + (long long)k * a.sz + (long long)gy * a.nx;
 #pragma unroll
                     for (int h = 0; h < H; ++h) {
@@ -785,8 +790,13 @@ __global__ __launch_bounds__((rowc_max_threads<R, CX, T>())) void k_rowc(
             if (out_plane && act) {
                 if constexpr (MODE == RM_SWEEP) {
                     T res[CX];
+                    bool odd = false;
 #pragma unroll
-                    for (int c = 0; c < CX; ++c) res[c] = finish<OP>(part[rp][c], ring[rp][c], kc);
+                    for (int c = 0; c < CX; ++c) res[c] = finish_fast<OP>(part[rp][c], ring[rp][c], kc, odd);
+                    if (OP == OP_THESIS && __builtin_expect(__any(odd), 0)) {
+#pragma unroll
+                        for (int c = 0; c < CX; ++c) res[c] = finish<OP>(part[rp][c], ring[rp][c], kc);
+                    }
                     T *row = static_cast<T *>(out_) + (long long)k * a.sz + (long long)gy * a.nx + xo;
                     if (whole || eqs) {
                         // equal shells: shell cells with the value they

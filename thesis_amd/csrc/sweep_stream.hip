@@ -377,9 +377,15 @@ __device__ __forceinline__ void sm_finish(SmPlane<CX, RPW> &out, const SmPlane<C
 {
     typedef float V4 __attribute__((ext_vector_type(4)));
 #pragma unroll
-    for (int r = 0; r < RPW; ++r)
+    for (int r = 0; r < RPW; ++r) {
+        bool odd = false;
 #pragma unroll
-        for (int c = 0; c < CX; ++c) out.v[r][c] = finish<OP>(part.v[r][c] + zp.v[r][c], cen.v[r][c], kc);
+        for (int c = 0; c < CX; ++c) out.v[r][c] = finish_fast<OP>(part.v[r][c] + zp.v[r][c], cen.v[r][c], kc, odd);
+        if (OP == OP_THESIS && __builtin_expect(__any(odd), 0)) {
+#pragma unroll
+            for (int c = 0; c < CX; ++c) out.v[r][c] = finish<OP>(part.v[r][c] + zp.v[r][c], cen.v[r][c], kc);
+        }
+    }
     if (zshell) {
         if (SH1 && (k == 0 || k == a.nz - 1)) {
             // a z-shell plane: u2's values (twice per z column of tiles)

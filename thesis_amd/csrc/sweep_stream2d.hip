@@ -100,12 +100,18 @@ __global__ __launch_bounds__(256) void k_stream2d(const float *__restrict__ X, f
             const bool yin = q >= 1 && q < a.ny - 1;
             const float xp = s2_prev_lane(v[7]);
             const float xn = s2_next_lane(v[0]);
-            float out[8], np[8];
+            float out[8], np[8], fin[8];
+            // row q: its sum plus the j-next term (row q+1 = v)
+            bool odd = false;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) fin[c] = finish_fast<OP>(part[l][c] + v[c], prev[l][c], kc, odd);
+            if (OP == OP_THESIS && __builtin_expect(__any(odd), 0)) {
+#pragma unroll
+                for (int c = 0; c < 8; ++c) fin[c] = finish<OP>(part[l][c] + v[c], prev[l][c], kc);
+            }
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
-                // row q: its sum plus the j-next term (row q+1 = v)
-                const float fin = finish<OP>(part[l][c] + v[c], prev[l][c], kc);
-                out[c] = (yin && ((xin >> c) & 1u)) ? fin : prev[l][c];
+                out[c] = (yin && ((xin >> c) & 1u)) ? fin[c] : prev[l][c];
                 // row q+1: i-prev, i-next, j-prev
                 float s = 0.0f;
                 s += c > 0 ? v[c - 1] : xp;
