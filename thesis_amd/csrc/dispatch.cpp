@@ -191,6 +191,7 @@ static st_status resolve(const st_params *p, Cfg &c, bool mixed)
     c.wy_d = c.core_d = c.zchunk_d = c.lds_d = 0;
     c.shell_eq = nullptr;
     c.block_steps = 0;
+    c.roll_steps = 0;
     c.resident = 0;
     c.zchunk = 0;
     c.lds = 0;
@@ -252,10 +253,12 @@ static st_status resolve(const st_params *p, Cfg &c, bool mixed)
             c.variant = march_ok ? ST_V_SMEM_REGISTER : ST_V_BASE;
             if (!march_ok) c.cx = 1;
         }
-        // 2D grids of radius 1 fuse sweeps per launch whichever family the
-        // rules above name (that family still serves stencil_sweep)
+        // 2D grids fuse sweeps per launch (radius 1) or march whole rows
+        // (radius 2 and up) whichever family the rules above name (that
+        // family still serves stencil_sweep)
         if (c.form == 0 && p->temporal_steps == 0) {
             resolve_block(c);
+            resolve_roll(c);
             // small 3D grids of radius 1: every sweep in one launch
             c.resident = resident_eligible(c, 1);
         }
@@ -344,6 +347,10 @@ st_status stencil_launch_config(const st_params *p, st_launch_info *info)
             info->temporal_steps = c.block_steps;
             info->launches = block_launches(c);
         }
+        if (c.roll_steps) {
+            info->temporal_steps = c.roll_steps;
+            info->launches = roll_launches(c);
+        }
         if (c.resident) {
             info->temporal_steps = c.iters;
             info->launches = 1;
@@ -390,6 +397,8 @@ st_status stencil_dispatch(const st_params *p, void *d_u1, void *d_u2, void *str
             // done, or failed
         } else if (c.block_steps) {
             s = run_block(c, d_u1, d_u2, hs, &in_u2);
+        } else if (c.roll_steps) {
+            s = run_roll(c, d_u1, d_u2, hs, &in_u2);
         } else if (c.variant == ST_V_COOP) {
             s = run_coop(c, d_u1, d_u2, hs, &in_u2);
         } else {

@@ -35,6 +35,7 @@ struct Cfg {
     int zchunk_d, lds_d; // frame differs): wave rows, core rows, z chunk, LDS bytes
     int resident;        // AUTO: the resident form runs the dispatch
     int block_steps;     // AUTO: sweeps per launch of the block form (0: not used)
+    int roll_steps;      // AUTO: sweeps per launch of the rolling form (0: not used)
     const int *shell_eq; // device flag: both buffers' shells hold the same bits
                          // (row form stores whole rows then); null: unknown
 };
@@ -104,6 +105,11 @@ st_status launch_rows_defect(const Cfg &c, bool f16, const float *x, const uint1
 // as single sweeps leave them.
 void resolve_block(Cfg &c);        // sets c.block_steps (0 where it is not taken)
 int block_launches(const Cfg &c);
+// AUTO's rolling form of 2D wide stars (sweep_roll.hip); sets c.roll_steps
+// (0 where it is not taken).
+void resolve_roll(Cfg &c);
+int roll_launches(const Cfg &c);
+st_status run_roll(const Cfg &c, void *u1, void *u2, hipStream_t s, int *in_u2);
 st_status run_block(const Cfg &c, void *u1, void *u2, hipStream_t s, int *in_u2);
 
 // Resident form, every sweep in one cooperative launch with the field in
