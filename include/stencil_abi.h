@@ -170,9 +170,9 @@ typedef struct st_launch_info {
     int grid_x, grid_y, grid_z;
     int coarsen_x, coarsen_y;
     int zchunk;                  /* planes per workgroup (SMEM_REGISTER)       */
-    int temporal_steps;          /* sweeps per pass (COOP; AUTO on 2D grids of
-                                    radius 1, which fuses sweeps whichever
-                                    single-sweep family `variant` names)       */
+    int temporal_steps;          /* sweeps per pass (COOP; AUTO on 2D grids,
+                                    which fuses sweeps whichever single-sweep
+                                    family `variant` names)                    */
     int lds_bytes;               /* LDS per workgroup                          */
     int launches;                /* sweep-kernel launches for `iterations`
                                     sweeps (the shell comparison and the

@@ -244,10 +244,11 @@ static st_status resolve(const st_params *p, Cfg &c, bool mixed)
             c.variant = ST_V_BASE;
             c.cx = 1;
         } else {
-            // FP32 up to radius 14, FP64 up to 8 in 3D (us per sweep, plain /
-            // this: FP32 320x256x256 R=14 602 / 311, R=16 394 / 1206; FP64
-            // 192^3 R=3 86 / 25, R=8 125 / 110, R=12 189 / 227)
-            const bool march_ok = c.dims == 3 ? c.r <= (c.dtype == ST_F64 ? 8 : 14)
+            // 3D: FP32 up to radius 14, FP64 up to 8, and where the tile form
+            // is ahead (us per sweep, plain / this: FP32 320x256x256 R=14
+            // 602 / 311, 384^3 R=16 805 / 301; FP64 192^3 R=3 86 / 25, R=9
+            // 138 / 75; the register march of radius 16 is behind, 394 / 1206)
+            const bool march_ok = c.dims == 3 ? c.r <= (c.dtype == ST_F64 ? 8 : 14) || tile_eligible(c)
                                               : (c.dtype == ST_F32 && c.r <= 8) ||
                                                     (c.dtype == ST_F64 && (c.r == 1 || c.r == 2 || c.r == 4));
             c.variant = march_ok ? ST_V_SMEM_REGISTER : ST_V_BASE;
