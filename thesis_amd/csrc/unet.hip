@@ -692,9 +692,9 @@ __global__ void k_bf16_to_f32(const bf16_t *__restrict__ a, float *__restrict__ 
 // 2 TB/s.  They take V channels per thread (16-byte loads and stores; V = 1
 // for channel counts or addresses that do not allow it), and a workgroup is
 // laid out as V-channel groups by columns by rows, so that the only division
-// is a 32-bit one of the thread index.  Before and now, us: 6 samples of 64^3
+// is a 32-bit one of the thread index.  Before and now, us: 8 samples of 64^3
 // with 16 channels k_relu_bwd 95 -> 46, k_bias_grad 48 -> 13, k_head_fwd
-// 64 -> 14, k_head_bwd 97 -> 47; a training step of 6 samples of 64^3,
+// 64 -> 14, k_head_bwd 97 -> 47; a training step of 8 samples of 64^3,
 // both levels: k_up_fwd 363 -> 72, k_pool_bwd 147 -> 60, k_chan_copy
 // 202 -> 133, k_pool_fwd 36 -> 18 (k_up_bwd stays at 101 to 111, bound by
 // the strided gather of its eight children).
@@ -1497,7 +1497,7 @@ st_status st_nn_mse(const float *base, const float *y, const float *target, floa
 {
     long long P = (long long)N * n * n * n;
     long long blocks = (P + 255) / 256;
-    if (blocks > 512) blocks = 512;  // one serial atomic per block (6 samples of 64^3: 4096 blocks 56 us, now 32)
+    if (blocks > 512) blocks = 512;  // one serial atomic per block (8 samples of 64^3: 4096 blocks 56 us, now 32)
     hipLaunchKernelGGL(k_mse, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream), base,
                        y, target, g, loss, pred, N, n, scale);
     return hip_check(hipGetLastError(), "mse launch");
