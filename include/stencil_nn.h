@@ -27,10 +27,13 @@ int st_nn_kpad(int ci);
 st_status st_nn_conv3(const void *act, const void *w, const float *bias, void *out_bf16,
                       float *out_f32, int N, int D, int H, int W, int Ci, int Co, int relu,
                       int accumulate, void *stream);
-/* dW[co][k] += sum_p dY[p][co] X[p+off(tap)][ci]  (FP32).  With Co a multiple
- * of 4 and Ci up to about 160 the partial sums of the workgroups go through
- * the library's workspace (at most 32 MiB, kept per device and stream) and
- * are added in a fixed order; else atomically. */
+/* dW[co][k] += sum_p dY[p][co] X[p+off(tap)][ci]  (FP32).  Ci a multiple of 8.
+ * Up to 176 input channels the partial sums of the workgroups go through the
+ * library's workspace (at most 32 MiB, kept per device and stream) and are
+ * added in a fixed order; above, and where tiles of 16 x 4 x 2 positions
+ * would be mostly padding, they are added atomically (with W a multiple of 8
+ * and Ci, Co <= 128 after a channel-major copy of both operands in the
+ * workspace, P*(Ci+Co) 16-bit words). */
 st_status st_nn_conv3_wgrad(const void *x, const void *dy, float *dw, int N, int D, int H, int W,
                             int Ci, int Co, void *stream);
 /* backward-data weights: Wt[ci][tap'*Co + co] = W[co][(26 - tap')*Ci + ci] */

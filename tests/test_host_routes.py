@@ -1,0 +1,72 @@
+"""The library's host side where there is no GPU: which kernels a call
+launches, what it does when the runtime refuses something, under capture and
+from several threads.  Each case runs in its own process on a stand-in for the
+HIP runtime (tests/hostsim/hip_standin.cpp), whose kernels do nothing."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes as C, re, sys, threading, time
+sys.path.insert(0, {root!r})
+R = C.CDLL({lib!r}, mode=C.RTLD_GLOBAL)
+log, answer = [], {{}}   # (event, handle, size, thread); event -> result or function
+@C.CFUNCTYPE(C.c_int, C.c_char_p, C.c_void_p, C.c_size_t, C.POINTER(C.c_void_p))
+def hook(event, handle, size, args):
+    event = event.decode()
+    m = re.search(r"k_[a-z0-9_]+", event)
+    name = m.group(0).rstrip("0123456789") if m else event
+    if m: name = re.match(r"\\d+(k_\\w+)", event[re.search(r"\\d+k_", event).start():]).group(1)[:int(re.search(r"(\\d+)k_", event).group(1))]
+    log.append((name, handle, size, threading.get_ident()))
+    a = answer.get(name, 0)
+    return a(handle, size, args) if callable(a) else a
+R.standin_hook(hook)
+def kernels(): return [e[0] for e in log if e[0].startswith("k_")]
+import thesis_amd as st
+from thesis_amd import nn
+def auto(nx, ny, nz=None, **kw):
+    kw = dict(dict(op=1, variant="auto", heuristic=1, iterations=4), **kw)
+    return st.StencilParams.make(nx=nx, ny=ny, nz=nz or 1, dimensions=3 if nz else 2, **kw)
+A, B = 1 << 20, 1 << 40  # addresses of buffers that no kernel touches
+"""
+
+
+@pytest.fixture(scope="session")
+def host(tmp_path_factory, st):
+    lib = str(tmp_path_factory.mktemp("standin") / "libamdhip64.so.7")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-std=c++17", "-Wl,-soname,libamdhip64.so.7", "-o", lib,
+                    os.path.join(HERE, "hostsim", "hip_standin.cpp")], check=True)
+
+    def run(body):
+        script = PRELUDE.format(root=ROOT, lib=lib) + textwrap.dedent(body)
+        r = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return run
+
+
+def test_wgrad_forms(host):
+    """Wide inputs and channel counts that are no multiple of 4 stay on the
+    tiled weight gradient; tiles that are mostly padding and a handful of
+    positions go to the kernels without tiles."""
+    host("""
+    def route(shape, ci, co):
+        log.clear()
+        nn.conv3_wgrad(A, A, A, shape, ci, co)
+        return kernels()
+    TILE, ROWS, GATHER = ["k_conv3_wgrad_tile", "k_wgrad_reduce"], ["k_pc_transpose"] * 2 + ["k_conv3_wgrad_t"], ["k_conv3_wgrad"]
+    for ci, co in ((96, 32), (104, 16), (112, 64), (128, 36), (128, 128), (176, 32), (16, 6), (32, 1), (24, 18)):
+        for shape in ((8, 16, 16, 16), (8, 8, 8, 8), (2, 33, 33, 33)):
+            assert route(shape, ci, co) == TILE, (shape, ci, co, route(shape, ci, co))
+    assert route((1, 1, 1, 100000), 64, 64) == ROWS       # 1 of 16 rows of a tile, whole octets of positions
+    assert route((1, 20000, 1, 1), 64, 64) == GATHER      # 1 of 64 positions
+    assert route((1, 20000, 1, 1), 16, 16) == TILE
+    assert route((1, 2, 2, 8), 64, 64) == GATHER
+    assert route((1, 1, 1, 1000), 64, 64) == TILE
+    assert route((8, 16, 16, 16), 192, 32) == GATHER      # no tile fits
+    """)

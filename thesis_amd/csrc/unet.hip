@@ -16,8 +16,9 @@
 // the weights transposed and the taps mirrored (conv_wt_transpose); the
 // weight gradient is a second MFMA GEMM reducing over positions.  Both take
 // their operands from tiles staged in LDS (k_conv3_tile, k_conv3_wgrad_tile);
-// k_conv3 and k_conv3_wgrad, which load every operand from global memory,
-// serve the shapes whose tile does not fit.
+// k_conv3, k_conv3_wgrad and k_conv3_wgrad_t, which load every operand from
+// global memory, serve the shapes whose tile does not fit or is mostly
+// padding.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -501,6 +502,130 @@ __global__ __launch_bounds__(256) void k_conv3_wgrad(const bf16_t *__restrict__ 
     }
 }
 
+// ---------------------------------------------------------------- weight gradient, channel-major operands
+
+// The MFMA operands of the weight gradient run along positions (8
+// consecutive positions of one channel per lane), which channels-last
+// activations hold Ci values apart: the gather above issues one 2-byte load
+// per value.  When rows are a multiple of 8 positions, both operands are
+// first transposed to channel-major [C][P] copies, and then every operand is
+// one 16-byte load: the dY rows directly, the X rows of a tap with dx = -1
+// or +1 from two aligned loads joined by a 16-bit funnel shift (a group of 8
+// positions never crosses a row, so only its first or last value can fall
+// outside the row, and it is zeroed).
+
+// [P][C] -> [C][P] (16-bit words) through LDS, 64 positions per workgroup.
+constexpr int kTrMaxC = 128;
+__global__ __launch_bounds__(256) void k_pc_transpose(const bf16_t *__restrict__ src, bf16_t *__restrict__ dst,
+                                                      int P, int C)
+{
+    __shared__ bf16_t t[kTrMaxC * 66];
+    const long long p0 = (long long)blockIdx.x * 64;
+    const int np = (int)min(64LL, (long long)P - p0);
+    for (int i = threadIdx.x; i < np * C; i += 256) {
+        const int pp = i / C, c = i - pp * C;
+        t[c * 66 + pp] = src[p0 * C + i];
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 64 * C; i += 256) {
+        const int c = i >> 6, pp = i & 63;
+        if (pp < np) dst[(long long)c * P + p0 + pp] = t[c * 66 + pp];
+    }
+}
+
+__device__ __forceinline__ u32x4 load8u(const bf16_t *p) { return *reinterpret_cast<const u32x4 *>(p); }
+
+// dW[co][k] += sum_p dYt[co][p] * Xt[ci(k)][p + off(tap(k))]; the same
+// tiling as k_conv3_wgrad (rows = output channels, 16*NB weight columns,
+// 32 positions per MFMA, `pchunk` positions per wave, atomics at the end).
+// Requires W % 8 == 0 and pchunk % 32 == 0.
+template <int NB>
+__global__ __launch_bounds__(256) void k_conv3_wgrad_t(const bf16_t *__restrict__ Xt,
+                                                       const bf16_t *__restrict__ dYt,
+                                                       float *__restrict__ dW, ConvGeom g, int pchunk)
+{
+    const int lane = threadIdx.x & 63;
+    const int j = lane & 15, grp = lane >> 4;
+    const long long wave = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const int K = 27 * g.Ci;
+    const int nkt = (K + 16 * NB - 1) / (16 * NB);
+    const int nct = (g.Co + 15) / 16;
+    const long long nchunks = ((long long)g.P + pchunk - 1) / pchunk;
+    const long long total = nchunks * nkt * nct;
+    if (wave >= total) return;
+    const int kt = (int)(wave % nkt);
+    const long long r2 = wave / nkt;
+    const int ct = (int)(r2 % nct);
+    const int pc = (int)(r2 / nct);
+    const int co = ct * 16 + j;  // A-operand row of this lane
+    const long long HW = (long long)g.H * g.W;
+    const bf16_t *arow = dYt + (long long)min(co, g.Co - 1) * g.P;
+    int kk[NB], dz[NB], dy[NB], dx[NB];
+    const bf16_t *brow[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+        kk[nb] = kt * 16 * NB + nb * 16 + j;  // B-operand column of this lane
+        const int kc = kk[nb] < K ? kk[nb] : 0;
+        const int tap = kc / g.Ci;
+        const int ci = kc - tap * g.Ci;
+        dz[nb] = tap / 9 - 1;
+        dy[nb] = (tap / 3) % 3 - 1;
+        dx[nb] = tap % 3 - 1;
+        brow[nb] = Xt + (long long)ci * g.P;
+    }
+    f32x4 acc[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int pbeg = pc * pchunk, pend = min(pbeg + pchunk, g.P);
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    for (int ps = pbeg; ps < pend; ps += 32) {
+        // this lane group's 8 positions: one row segment (W % 8 == 0)
+        const int pf = ps + grp * 8;
+        const bool pin = pf < pend;
+        int n0, z0, y0, x0;
+        decode(g, min(pf, g.P - 8), n0, z0, y0, x0);
+        const u32x4 av = (pin && co < g.Co) ? load8u(arow + pf) : zero;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const int zz = z0 + dz[nb], yy = y0 + dy[nb];
+            const bool ok = pin && kk[nb] < K && zz >= 0 && zz < g.D && yy >= 0 && yy < g.H;
+            u32x4 b = zero;
+            if (ok) {
+                const bf16_t *q = brow[nb] + pf + (long long)dz[nb] * HW + (long long)dy[nb] * g.W;
+                const u32x4 v = load8u(q);
+                if (dx[nb] == 0) {
+                    b = v;
+                } else if (dx[nb] < 0) {
+                    // values x0-1 .. x0+6: the last of the group before, then v[0..6]
+                    const unsigned prev = x0 > 0 ? load8u(q - 8)[3] : 0u;
+                    b[0] = __builtin_amdgcn_alignbit(v[0], prev, 16);
+                    b[1] = __builtin_amdgcn_alignbit(v[1], v[0], 16);
+                    b[2] = __builtin_amdgcn_alignbit(v[2], v[1], 16);
+                    b[3] = __builtin_amdgcn_alignbit(v[3], v[2], 16);
+                } else {
+                    // values x0+1 .. x0+8: v[1..7], then the first of the group after
+                    const unsigned next = x0 + 8 < g.W ? load8u(q + 8)[0] : 0u;
+                    b[0] = __builtin_amdgcn_alignbit(v[1], v[0], 16);
+                    b[1] = __builtin_amdgcn_alignbit(v[2], v[1], 16);
+                    b[2] = __builtin_amdgcn_alignbit(v[3], v[2], 16);
+                    b[3] = __builtin_amdgcn_alignbit(next, v[3], 16);
+                }
+            }
+            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av),
+                                                              __builtin_bit_cast(bf16x8, b), acc[nb], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+        if (kk[nb] >= K) continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int c = ct * 16 + 4 * grp + e;
+            if (c < g.Co) atomicAdd(dW + (long long)c * g.Kpad + kk[nb], acc[nb][e]);
+        }
+    }
+}
+
 // ---------------------------------------------------------------- weight gradient, LDS tiles
 
 // dW[co][k] += sum_p dY[p][co] * X[p + off(tap)][ci] over tiles of 16 x 4 x
@@ -510,13 +635,15 @@ __global__ __launch_bounds__(256) void k_conv3_wgrad(const bf16_t *__restrict__ 
 // both operands run along positions, which channels-last data holds Ci apart:
 // ds_read_b64_tr_b16 reads four positions x 16 channels and hands each lane
 // one channel's four positions, and a tap is an address, not a shift.  (The
-// gathering kernel above reads two bytes at a time; channel-major copies of
-// both operands, with a 16-bit funnel shift for dx = -1 and +1 and one load
-// from L2 per operand, took 1407 us for 48 -> 16 channels at 8 x 64^3.)
+// channel-major kernel above, one load from L2 per operand, takes 1407 us
+// for 48 -> 16 channels at 8 x 64^3.)
 //
 // Wave w of WAVES owns the column blocks w, w + WAVES, .. (16 weight columns
 // k each) of 16*NC output channels and keeps their sums in registers over all
-// of its workgroup's tiles; every workgroup writes its partial dW to the
+// of its workgroup's tiles; above 96 input channels, where the registers no
+// longer hold all columns, workgroups share the columns out in ranges (8 x
+// 16^3 104 -> 16 gathering 327 us, channel-major 132, now 44; 128 -> 128 856,
+// 339, 163).  Every workgroup writes its partial dW to the
 // workspace, and k_wgrad_reduce adds them up in a fixed order.
 //
 // Bound: LDS reads (two 8-byte reads per lane for each B operand, used for
@@ -539,12 +666,15 @@ __device__ __forceinline__ bf16x8 read_tr(const char *p, int S4)
     return __builtin_bit_cast(bf16x8, v);
 }
 
-// NBW column blocks per wave (those below nkb exist), NC blocks of 16 output
-// channels from c0 = 16*NC*blockIdx.y
+// NBW column blocks per wave (those below nkb exist) of the range of `cols`
+// column blocks from cols*blockIdx.z, NC blocks of 16 output channels from
+// c0 = 16*NC*blockIdx.y.  wide: dY can be read four channels at a time (Co a
+// multiple of 4, 8-byte address).
 template <int NC, int NBW, int TZ>
 __global__ __launch_bounds__(64 * kWgWaves) void k_conv3_wgrad_tile(const bf16_t *__restrict__ X,
                                                                     const bf16_t *__restrict__ dY,
-                                                                    float *__restrict__ part, TileGeom q, int ntiles)
+                                                                    float *__restrict__ part, TileGeom q, int ntiles, int cols,
+                                                                    int wide)
 {
     extern __shared__ __align__(16) char lds[];
     const ConvGeom &g = q.g;
@@ -553,14 +683,15 @@ __global__ __launch_bounds__(64 * kWgWaves) void k_conv3_wgrad_tile(const bf16_t
     char *const ylds = lds + tile_positions(TZ) * S;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int grp = lane >> 4, c0 = 16 * NC * (int)blockIdx.y;
-    const int K = 27 * g.Ci, nkb = (K + 15) / 16;
+    const int K = 27 * g.Ci, kb0 = cols * (int)blockIdx.z, nkb = min(kb0 + cols, (K + 15) / 16);
+    const int wb = kb0 + w;  // the wave's first column block
     // the lane's place in a transposed read: positions 8*(grp & 1) + (lane & 15)/4
     // (+4) of row grp/2 of the step's two rows
     const int xr = 8 * (grp & 1) + ((lane & 15) >> 2);
     int boff[NBW];  // X: plus the tap and channel of the lane's four columns
 #pragma unroll
     for (int i = 0; i < NBW; ++i) {
-        const int k = min((w + i * kWgWaves) * 16 + 4 * (lane & 3), K - 4), tap = k / g.Ci;
+        const int k = min((wb + i * kWgWaves) * 16 + 4 * (lane & 3), K - 4), tap = k / g.Ci;
         boff[i] = ((grp >> 1) * (kTx + 2) + xr) * S + tap_offset(tap, k - tap * g.Ci, S);
     }
     const int aoff = ((grp >> 1) * kTx + xr) * SY + 8 * (lane & 3);
@@ -580,8 +711,14 @@ __global__ __launch_bounds__(64 * kWgWaves) void k_conv3_wgrad_tile(const bf16_t
             const int c4 = i % (NC * 4), p = i / (NC * 4), px = p % kTx, r = p / kTx;
             const int x = x0 + px, y = y0 + r % kTy, z = z0 + r / kTy, c = c0 + c4 * 4;
             uint2 v = make_uint2(0u, 0u);
-            if (x < g.W && y < g.H && z < g.D && c < g.Co)
-                v = *reinterpret_cast<const uint2 *>(dY + (sample + ((long long)z * g.H + y) * g.W + x) * g.Co + c);
+            if (x < g.W && y < g.H && z < g.D && c < g.Co) {
+                const bf16_t *src = dY + (sample + ((long long)z * g.H + y) * g.W + x) * g.Co + c;
+                if (wide) v = *reinterpret_cast<const uint2 *>(src);
+                else {
+                    v.x = src[0] | (c + 1 < g.Co ? (unsigned)src[1] << 16 : 0u);
+                    v.y = (c + 2 < g.Co ? (unsigned)src[2] : 0u) | (c + 3 < g.Co ? (unsigned)src[3] << 16 : 0u);
+                }
+            }
             *reinterpret_cast<uint2 *>(ylds + p * SY + c4 * 8) = v;
         }
         __syncthreads();
@@ -606,7 +743,7 @@ __global__ __launch_bounds__(64 * kWgWaves) void k_conv3_wgrad_tile(const bf16_t
             }
 #pragma unroll
             for (int i = 0; i < NBW; ++i) {
-                if (w + i * kWgWaves >= nkb) break;
+                if (wb + i * kWgWaves >= nkb) break;
                 bf16x8 b = read_tr(xp + boff[i], 4 * S);
                 if (edge) b = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, b) & keep);
 #pragma unroll
@@ -620,8 +757,8 @@ __global__ __launch_bounds__(64 * kWgWaves) void k_conv3_wgrad_tile(const bf16_t
     float *const o = part + (long long)blockIdx.x * g.Co * g.Kpad;
 #pragma unroll
     for (int i = 0; i < NBW; ++i) {
-        const int k = (w + i * kWgWaves) * 16 + (lane & 15);
-        if (k >= K) continue;
+        const int k = (wb + i * kWgWaves) * 16 + (lane & 15);
+        if (k >= min(16 * nkb, K)) continue;
 #pragma unroll
         for (int c = 0; c < NC; ++c)
 #pragma unroll
@@ -1236,13 +1373,15 @@ static ConvTilePlan conv_tile_plan(const ConvGeom &g, const void *out_bf, const 
     return t;
 }
 
-// The tiled weight gradient of a layer (fn null: none): parts workgroups per
-// group of 16*NC output channels.
+// The tiled weight gradient of a layer (fn null: none).
 struct WgradTilePlan {
     const void *fn = nullptr;
     TileGeom q;
-    int ntiles, parts, groups, lds;
+    int ntiles, positions;   // tiles, positions of a tile
+    int parts, groups;       // workgroups per group of 16*NC output channels
+    int ranges, cols, lds;   // ranges of `cols` column blocks
 };
+constexpr int kWgMaxBlocks = 21;  // column blocks of a wave, the most its registers hold (Ci = 96)
 
 template <int NC, int TZ>
 static const void *wgrad_tile_fn(int nbw)
@@ -1259,9 +1398,12 @@ static const void *wgrad_tile_fn(int nbw)
 static WgradTilePlan wgrad_tile_plan(const ConvGeom &g)
 {
     WgradTilePlan t;
-    if (g.Co % 4 || g.Co < 4) return t;  // dY is read four channels at a time
     const int nc = g.Co > 16 ? 2 : 1;
-    const int nbw = ((27 * g.Ci + 15) / 16 + kWgWaves - 1) / kWgWaves;
+    // ranges of weight columns of at most kWgMaxBlocks blocks per wave
+    const int nkb = (27 * g.Ci + 15) / 16;
+    t.ranges = (nkb + kWgMaxBlocks * kWgWaves - 1) / (kWgMaxBlocks * kWgWaves);
+    t.cols = (nkb + t.ranges - 1) / t.ranges;
+    const int nbw = (t.cols + kWgWaves - 1) / kWgWaves;
     // tiles of 4 planes while two workgroups fit a CU's LDS, else of 2
     auto lds = [&](int tz) { return tile_positions(tz) * tile_stride(g.Ci) + tz * kTy * kTx * (nc * 32 + (nc == 1 ? 0 : 16)); };
     const int tz = lds(4) <= 80 * 1024 ? 4 : 2;
@@ -1274,13 +1416,39 @@ static WgradTilePlan wgrad_tile_plan(const ConvGeom &g)
     const long long tiles = (long long)g.N * t.q.tx * t.q.ty * t.q.tz;
     if (tiles >= (1LL << 31)) return t;
     t.ntiles = (int)tiles;
+    t.positions = tz * kTy * kTx;
     t.groups = (g.Co + 16 * nc - 1) / (16 * nc);
-    // two workgroups per CU, and at most 32 MiB of partial sums
-    const long long want = std::min(512LL / t.groups, (32LL << 20) / (4LL * g.Co * g.Kpad));
+    if (t.groups > 65535) return t;
+    // one round of workgroups at most (one or two per CU, as their LDS lets
+    // them) and 32 MiB of partial sums, which leaves 101 of 256 CUs at work for
+    // 96 -> 32 channels and 150 for 64 -> 64
+    const long long round = t.lds > kMaxLds / 2 ? 256 : 512;
+    const long long want = std::min(round / (t.groups * t.ranges), (32LL << 20) / (4LL * g.Co * g.Kpad));
     t.parts = (int)std::max(1LL, std::min((long long)t.ntiles, want));
     if (nc == 1) t.fn = tz == 4 ? wgrad_tile_fn<1, 4>(nbw) : wgrad_tile_fn<1, 2>(nbw);
     else t.fn = tz == 4 ? wgrad_tile_fn<2, 4>(nbw) : wgrad_tile_fn<2, 2>(nbw);
     return t;
+}
+
+enum WgradForm { WG_TILE = 1, WG_CHANNEL_MAJOR, WG_GATHER };
+
+// Where tiles are mostly padding and there are many of them, the kernels that
+// flatten positions are ahead (us, tiles / channel-major rows / gathering:
+// 1 x 1 x 1 x 100000 positions 64 -> 64 channels 570 / 185 / 527, 4000 x 2 x 2
+// x 2 128 -> 128 1517 / - / 688, but 16 -> 16 few products and 1 x 1 x 1 x 1000
+// 64 -> 64 few tiles: 20 / 66 / 151), and a handful of positions is one step
+// of the gathering kernel (1 x 2 x 2 x 2 64 -> 64 16.5 / - / 8.1).
+static WgradForm wgrad_form(const ConvGeom &g, const WgradTilePlan &t)
+{
+    const bool rows = g.W % 8 == 0 && g.Ci <= kTrMaxC && g.Co <= kTrMaxC;
+    const WgradForm flat = rows ? WG_CHANNEL_MAJOR : WG_GATHER;
+    if (!t.fn) return flat;
+    if (g.P <= (g.Ci >= 32 ? 64 : 32)) return WG_GATHER;
+    const long long room = (long long)t.ntiles * t.positions, P = g.P;
+    // rows of positions alone: 18 of 27 taps lie outside and cost no load
+    const int least = rows || (g.D == 1 && g.H == 1) ? 8 : 16;
+    if (t.ntiles >= 1024 && least * P <= room && (rows || g.Ci * g.Co >= 1536)) return flat;
+    return WG_TILE;
 }
 
 extern "C" {
@@ -1324,15 +1492,18 @@ st_status st_nn_conv3_wgrad(const void *x, const void *dy, float *dw, int N, int
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bf16_t *xb = static_cast<const bf16_t *>(x), *yb = static_cast<const bf16_t *>(dy);
     const WgradTilePlan t = wgrad_tile_plan(g);
-    if (t.fn) {
+    const WgradForm form = wgrad_form(g, t);
+    if (form == WG_TILE) {
         void *ws = nullptr;
         st_status st = workspace_slot(0, (size_t)t.parts * Co * g.Kpad * sizeof(float), s, &ws);
         if (st != ST_OK) return st;
         float *part = static_cast<float *>(ws);
-        void *args[] = {&xb, &yb, &part, const_cast<TileGeom *>(&t.q), const_cast<int *>(&t.ntiles)};
+        int wide = Co % 4 == 0 && (reinterpret_cast<uintptr_t>(dy) & 7) == 0;
+        void *args[] = {&xb, &yb, &part, const_cast<TileGeom *>(&t.q), const_cast<int *>(&t.ntiles), const_cast<int *>(&t.cols),
+                        &wide};
         hipError_t e = hipFuncSetAttribute(t.fn, hipFuncAttributeMaxDynamicSharedMemorySize, t.lds);
         if (e != hipSuccess) return hip_check(e, "hipFuncSetAttribute(wgrad LDS)");
-        e = hipLaunchKernel(t.fn, dim3(t.parts, t.groups), dim3(64 * kWgWaves), args, t.lds, s);
+        e = hipLaunchKernel(t.fn, dim3(t.parts, t.groups, t.ranges), dim3(64 * kWgWaves), args, t.lds, s);
         if (e != hipSuccess) return hip_check(e, "conv3 wgrad launch");
         const int n = Co * g.Kpad;
         hipLaunchKernelGGL(k_wgrad_reduce, dim3((n + 63) / 64), dim3(256), 0, s, part, dw, n, 27 * Ci, g.Kpad, t.parts);
@@ -1343,6 +1514,18 @@ st_status st_nn_conv3_wgrad(const void *x, const void *dy, float *dw, int N, int
     const long long nkt = (K + 63) / 64, nct = (Co + 15) / 16, nch = (g.P + pchunk - 1) / pchunk;
     const long long waves = nkt * nct * nch;
     const dim3 grid((unsigned)((waves + 3) / 4));
+    if (form == WG_CHANNEL_MAJOR) {
+        // channel-major copies of both operands in the workspace (slot 0)
+        void *ws = nullptr;
+        st_status st = workspace_slot(0, ((size_t)g.P * Ci + (size_t)g.P * Co) * sizeof(bf16_t), s, &ws);
+        if (st != ST_OK) return st;
+        bf16_t *xt = static_cast<bf16_t *>(ws), *dyt = xt + (size_t)g.P * Ci;
+        const dim3 tg((unsigned)((g.P + 63) / 64));
+        hipLaunchKernelGGL(k_pc_transpose, tg, dim3(256), 0, s, xb, xt, g.P, Ci);
+        hipLaunchKernelGGL(k_pc_transpose, tg, dim3(256), 0, s, yb, dyt, g.P, Co);
+        hipLaunchKernelGGL((k_conv3_wgrad_t<4>), grid, dim3(256), 0, s, xt, dyt, dw, g, pchunk);
+        return hip_check(hipGetLastError(), "conv3 wgrad launch");
+    }
     hipLaunchKernelGGL((k_conv3_wgrad<4>), grid, dim3(256), 0, s, xb, yb, dw, g, pchunk);
     return hip_check(hipGetLastError(), "conv3 wgrad launch");
 }
