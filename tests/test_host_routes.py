@@ -70,3 +70,21 @@ def test_wgrad_forms(host):
     assert route((1, 1, 1, 1000), 64, 64) == TILE
     assert route((8, 16, 16, 16), 192, 32) == GATHER      # no tile fits
     """)
+
+
+def test_conv_forms(host):
+    """The tiled convolution where its tiles are filled and fill the card, the
+    kernel without tiles elsewhere."""
+    host("""
+    def route(shape, ci, co):
+        log.clear()
+        nn.conv3(A, A, A, A, None, shape, ci, co)
+        return kernels()
+    for shape, ci, co in (((8, 64, 64, 64), 48, 16), ((8, 64, 64, 64), 16, 48), ((8, 16, 16, 16), 64, 64),
+                          ((8, 32, 32, 32), 96, 32), ((8, 32, 32, 32), 64, 64), ((4, 4, 4, 4), 16, 16), ((1, 2, 2, 2), 8, 16)):
+        assert route(shape, ci, co) == ["k_conv3_tile"], (shape, ci, co)
+    for shape, ci, co in (((1, 1, 1, 100000), 16, 16), ((1, 300, 300, 3), 64, 64), ((4, 20, 20, 20), 128, 128),
+                          ((1, 40, 40, 40), 64, 80), ((8, 32, 32, 32), 64, 80), ((64, 8, 8, 8), 64, 256),
+                          ((4000, 2, 2, 2), 8, 16), ((1, 1, 300, 301), 32, 32)):
+        assert route(shape, ci, co) == ["k_conv3"], (shape, ci, co)
+    """)

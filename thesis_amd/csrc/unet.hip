@@ -642,8 +642,8 @@ __global__ __launch_bounds__(256) void k_conv3_wgrad_t(const bf16_t *__restrict_
 // k each) of 16*NC output channels and keeps their sums in registers over all
 // of its workgroup's tiles; above 96 input channels, where the registers no
 // longer hold all columns, workgroups share the columns out in ranges (8 x
-// 16^3 104 -> 16 gathering 327 us, channel-major 132, now 44; 128 -> 128 856,
-// 339, 163).  Every workgroup writes its partial dW to the
+// 16^3 104 -> 16 gathering 327 us, channel-major 132, now 31; 128 -> 128 856,
+// 339, 164).  Every workgroup writes its partial dW to the
 // workspace, and k_wgrad_reduce adds them up in a fixed order.
 //
 // Bound: LDS reads (two 8-byte reads per lane for each B operand, used for
@@ -1346,6 +1346,31 @@ static const void *conv_tile_fn(int mb)
                    : reinterpret_cast<const void *>(&k_conv3_tile<NB, 2>);
 }
 
+// blocks of 16 output channels of a wave of k_conv3
+static int conv_flat_nb(int co) { return co >= 64 ? 4 : (co >= 32 ? 2 : 1); }
+
+// Whether the tiles are ahead of k_conv3, by the time a chunk of 32 weight
+// columns takes in each (us, fitted to 690 shapes of 8 to 262144 positions and
+// 4 to 256 channels; the choice is within 1% of the better one on average, at
+// worst 1.2 times).  Tiles: per round of workgroups, by channel blocks, depth
+// and workgroups per CU.  k_conv3: a latency until the waves fill the card,
+// then a rate; taps outside a sample of one plane, row or column cost it no
+// load.  64 -> 64 channels, tiles / k_conv3: 8 x 16^3 31 / 64, 1 x 40^3
+// 83 / 69; 64 -> 80 (channel blocks in two halves, each staging the tile)
+// 135 / 91; 1 x 300 x 300 x 3 (3 of 16 columns) 1136 / 232.
+static bool conv_tile_ahead(const ConvGeom &g, int nb, int mb, bool two_per_cu, int blocks)
+{
+    static const double tile[4][2] = {{0.19, 0.36}, {0.29, 0.45}, {0.32, 0.70}, {0.43, 0.60}};
+    const long long round = two_per_cu ? 512 : 256;
+    double t = (double)((blocks + round - 1) / round) * tile[nb - 1][mb == 4 || (nb == 4 && two_per_cu)];
+    if ((g.Co + 15) / 16 % nb) t *= 1.2;  // a last group of fewer blocks
+    const int fb = conv_flat_nb(g.Co);
+    const double waves = (double)((g.P + 63) / 64) * ((g.Co + 16 * fb - 1) / (16 * fb)) / 1024;
+    double f = fb == 1 ? std::max(0.95, 0.50 * waves) : fb == 2 ? std::max(0.85, 0.60 * waves) : std::max(1.15, 0.87 * waves);
+    if (g.D == 1 || g.H == 1 || g.W == 1) f *= 0.7;
+    return t <= f;
+}
+
 static ConvTilePlan conv_tile_plan(const ConvGeom &g, const void *out_bf, const void *out_f)
 {
     ConvTilePlan t;
@@ -1367,7 +1392,7 @@ static ConvTilePlan conv_tile_plan(const ConvGeom &g, const void *out_bf, const 
     t.q.ty = (g.H + kTy - 1) / kTy;
     t.q.tz = (g.D + mb - 1) / mb;
     const long long blocks = (long long)g.N * t.q.tx * t.q.ty * t.q.tz * t.nct;
-    if (blocks >= (1LL << 31)) return t;
+    if (blocks >= (1LL << 31) || !conv_tile_ahead(g, nb, mb, t.lds <= kMaxLds / 2, (int)blocks)) return t;
     t.blocks = (int)blocks;
     t.fn = nb == 4 ? conv_tile_fn<4>(mb) : nb == 3 ? conv_tile_fn<3>(mb) : nb == 2 ? conv_tile_fn<2>(mb) : conv_tile_fn<1>(mb);
     return t;
@@ -1474,7 +1499,7 @@ st_status st_nn_conv3(const void *act, const void *w, const float *bias, void *o
         if (e != hipSuccess) return hip_check(e, "hipFuncSetAttribute(conv3 LDS)");
         return hip_check(hipLaunchKernel(t.fn, dim3(t.blocks), dim3(256), args, t.lds, s), "conv3 launch");
     }
-    const int nb = Co >= 64 ? 4 : (Co >= 32 ? 2 : 1);
+    const int nb = conv_flat_nb(Co);
     const long long waves = ((g.P + 63) / 64) * ((Co + 16 * nb - 1) / (16 * nb));
     const dim3 grid((unsigned)((waves + 3) / 4)), block(256);
     if (nb == 4) hipLaunchKernelGGL((k_conv3<4, 4>), grid, block, 0, s, a, wt, bias, ob, out_f32, g, relu, accumulate);
