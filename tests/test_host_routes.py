@@ -88,3 +88,15 @@ def test_conv_forms(host):
                           ((4000, 2, 2, 2), 8, 16), ((1, 1, 300, 301), 32, 32)):
         assert route(shape, ci, co) == ["k_conv3"], (shape, ci, co)
     """)
+
+
+def test_mixed_small_kernels(host):
+    """The 16-bit modes off the row kernels: one flat kernel per pass."""
+    host("""
+    p = auto(17, 300, 300, radius=4, dtype=st.BF16, iterations=3, restart=10)
+    sizes = []
+    answer["k_mx_sweep"] = lambda stream, size, args: sizes.append(size) or 0
+    st.dispatch_mixed(p, A, A, A, A, A)
+    cells = 9 * 292 * 292
+    assert kernels().count("k_mx_defect") == 1 and sizes == [-(-cells // 256)] * 3, (kernels(), sizes)
+    """)

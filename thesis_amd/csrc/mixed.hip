@@ -10,8 +10,6 @@
 // Every `restart` sweeps the correction is folded into x in FP32 and the
 // defect is recomputed in FP32 from the new x (the FP32-residual defect
 // correction); 16-bit rounding then only ever applies to increments.
-#include <algorithm>
-
 #include "st_device.hpp"
 #include "st_half.hpp"
 #include "st_internal.hpp"
@@ -24,85 +22,74 @@ struct MixArgs {
     float w;
 };
 
-// The per-cell kernels, for the grids the row-streaming kernels do not take
-// (2D, widths that are no multiple of 4, radii above 4).  Bound: the
-// 2-byte loads of a cell's 4R or 6R neighbours, one instruction each; a
-// workgroup of 64 x 4 threads has them all in flight (radius 1 to 4 unrolled,
-// RS = 0: any) and finds its cell without the 64-bit divisions of a linear
-// index, which with one load after the other took 34 us a sweep of 123x284x71
-// R = 4, now @MX@.
-//
-// f(index) for every interior cell.
-template <typename F>
-__device__ __forceinline__ void each_interior(const MixArgs &a, F f)
+// Decompose interior index t into (i, j, k).
+__device__ __forceinline__ long long interior_idx(const MixArgs &a, long long t)
 {
     const Geom &g = a.g;
-    const int R = g.r, k0 = a.dims == 3 ? R : 0, k1 = a.dims == 3 ? g.nz - R : 1;
-    for (int k = k0 + (int)blockIdx.z; k < k1; k += (int)gridDim.z)
-        for (long long j = R + (long long)blockIdx.y * 4 + (threadIdx.x >> 6); j < g.ny - R; j += 4LL * gridDim.y)
-            for (long long i = R + (long long)blockIdx.x * 64 + (threadIdx.x & 63); i < g.nx - R; i += 64LL * gridDim.x)
-                f(i + j * g.sy + k * g.sz);
+    const int R = g.r;
+    const int wx = g.nx - 2 * R, wy = g.ny - 2 * R;
+    const long long wxy = (long long)wx * wy;
+    const int kk = (int)(t / wxy);
+    const long long rem = t - (long long)kk * wxy;
+    const int j = R + (int)(rem / wx);
+    const int i = R + (int)(rem - (long long)(j - R) * wx);
+    const int k = a.dims == 3 ? R + kk : 0;
+    return i + j * g.sy + k * g.sz;
 }
 
-// Sum of the neighbours of p[0] in the reference's order, v(neighbour) each.
-template <int RS, typename T, typename V>
-__device__ __forceinline__ float neighbour_sum(const T *p, const MixArgs &a, V v)
+__device__ __forceinline__ long long interior_count(const MixArgs &a)
 {
-    const int R = RS ? RS : a.g.r;
-    float s = 0.0f;
-    auto axis = [&](long long st) {
-#pragma unroll
-        for (int q = R; q >= 1; --q) s += v(p[-q * st]);
-#pragma unroll
-        for (int q = 1; q <= R; ++q) s += v(p[q * st]);
-    };
-    axis(1);
-    axis(a.g.sy);
-    if (a.dims == 3) axis(a.g.sz);
-    return s;
+    const Geom &g = a.g;
+    const int R = g.r;
+    return (long long)(g.nx - 2 * R) * (g.ny - 2 * R) * (a.dims == 3 ? g.nz - 2 * R : 1);
 }
 
 // d = round16(G(x) - x) on the interior; G is the FP32 JACOBI cell.
-template <bool F16, int RS>
-__global__ __launch_bounds__(256) void k_mx_defect(const float *__restrict__ x, uint16_t *__restrict__ d, MixArgs a)
+template <bool F16>
+__global__ __launch_bounds__(256) void k_mx_defect(const float *__restrict__ x,
+                                                   uint16_t *__restrict__ d, MixArgs a)
 {
-    each_interior(a, [&](long long idx) {
-        const float tcell = neighbour_sum<RS>(x + idx, a, [](float q) { return q; }) * a.w;
+    const Geom &g = a.g;
+    const int R = g.r;
+    const long long n = interior_count(a), stride = (long long)gridDim.x * blockDim.x;
+    for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < n; t += stride) {
+        const long long idx = interior_idx(a, t);
+        float u = 0.0f;
+        for (int q = R; q >= 1; --q) u += x[idx - q];
+        for (int q = 1; q <= R; ++q) u += x[idx + q];
+        for (int q = R; q >= 1; --q) u += x[idx - q * g.sy];
+        for (int q = 1; q <= R; ++q) u += x[idx + q * g.sy];
+        if (a.dims == 3) {
+            for (int q = R; q >= 1; --q) u += x[idx - q * g.sz];
+            for (int q = 1; q <= R; ++q) u += x[idx + q * g.sz];
+        }
+        const float tcell = u * a.w;
         d[idx] = rnd16<F16>(tcell - x[idx]);
-    });
+    }
 }
 
 // e' = round16(widen(d) + w * sum widen(e neighbours)).
-template <bool F16, int RS>
-__global__ __launch_bounds__(256) void k_mx_sweep(const uint16_t *__restrict__ e, const uint16_t *__restrict__ d,
+template <bool F16>
+__global__ __launch_bounds__(256) void k_mx_sweep(const uint16_t *__restrict__ e,
+                                                  const uint16_t *__restrict__ d,
                                                   uint16_t *__restrict__ eo, MixArgs a)
 {
-    each_interior(a, [&](long long idx) {
-        const float sw = neighbour_sum<RS>(e + idx, a, [](uint16_t q) { return wid16<F16>(q); }) * a.w;
+    const Geom &g = a.g;
+    const int R = g.r;
+    const long long n = interior_count(a), stride = (long long)gridDim.x * blockDim.x;
+    for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < n; t += stride) {
+        const long long idx = interior_idx(a, t);
+        float s = 0.0f;
+        for (int q = R; q >= 1; --q) s += wid16<F16>(e[idx - q]);
+        for (int q = 1; q <= R; ++q) s += wid16<F16>(e[idx + q]);
+        for (int q = R; q >= 1; --q) s += wid16<F16>(e[idx - q * g.sy]);
+        for (int q = 1; q <= R; ++q) s += wid16<F16>(e[idx + q * g.sy]);
+        if (a.dims == 3) {
+            for (int q = R; q >= 1; --q) s += wid16<F16>(e[idx - q * g.sz]);
+            for (int q = 1; q <= R; ++q) s += wid16<F16>(e[idx + q * g.sz]);
+        }
+        const float sw = s * a.w;
         eo[idx] = rnd16<F16>(wid16<F16>(d[idx]) + sw);
-    });
-}
-
-template <bool F16, int RS>
-static void mx_launch(const MixArgs &a, dim3 grid, const float *x, const uint16_t *e, uint16_t *d, uint16_t *eo, hipStream_t s)
-{
-    if (x) hipLaunchKernelGGL((k_mx_defect<F16, RS>), grid, dim3(256), 0, s, x, d, a);
-    else hipLaunchKernelGGL((k_mx_sweep<F16, RS>), grid, dim3(256), 0, s, e, d, eo, a);
-}
-
-// The defect of x, or where x is null the sweep e -> eo.
-template <bool F16>
-static void mx_cells(const MixArgs &a, const float *x, const uint16_t *e, uint16_t *d, uint16_t *eo, hipStream_t s)
-{
-    auto blocks = [](long long n, long long per) { return (unsigned)std::max(1LL, std::min((n + per - 1) / per, 65535LL)); };
-    const int R = a.g.r;
-    const dim3 grid(blocks(a.g.nx - 2 * R, 64), blocks(a.g.ny - 2 * R, 4), blocks(a.dims == 3 ? a.g.nz - 2 * R : 1, 1));
-    switch (R) {
-    case 1: return mx_launch<F16, 1>(a, grid, x, e, d, eo, s);
-    case 2: return mx_launch<F16, 2>(a, grid, x, e, d, eo, s);
-    case 3: return mx_launch<F16, 3>(a, grid, x, e, d, eo, s);
-    case 4: return mx_launch<F16, 4>(a, grid, x, e, d, eo, s);
-    default: return mx_launch<F16, 0>(a, grid, x, e, d, eo, s);
     }
 }
 
@@ -169,6 +156,8 @@ static st_status mixed_impl(const Cfg &c, float *x, uint16_t *e1, uint16_t *e2, 
     a.dims = c.dims;
     a.w = (float)c.weight;
     const long long n = (long long)c.nx * c.ny * c.nz;
+    const int R = c.r;
+    const long long ni = (long long)(c.nx - 2 * R) * (c.ny - 2 * R) * (c.dims == 3 ? c.nz - 2 * R : 1);
     auto blocks = [](long long cnt) {
         long long b = (cnt + 255) / 256;
         if (b > 32768) b = 32768;
@@ -216,11 +205,11 @@ static st_status mixed_impl(const Cfg &c, float *x, uint16_t *e1, uint16_t *e2, 
     }
     auto defect = [&]() {
         if (rows) st = launch_rows_mixed(c, 1, F16, x, d, nullptr, s);
-        else mx_cells<F16>(a, x, nullptr, d, nullptr, s);
+        else hipLaunchKernelGGL(k_mx_defect<F16>, blocks(ni), dim3(256), 0, s, x, d, a);
     };
     auto sweep = [&](const uint16_t *ein, uint16_t *eout) {
         if (rows) st = launch_rows_mixed(c, 0, F16, ein, eout, d, s);
-        else mx_cells<F16>(a, nullptr, ein, d, eout, s);
+        else hipLaunchKernelGGL(k_mx_sweep<F16>, blocks(ni), dim3(256), 0, s, ein, d, eout, a);
     };
     defect();
     uint16_t *ea = e1, *eb = e2;
