@@ -100,3 +100,19 @@ def test_mixed_small_kernels(host):
     cells = 9 * 292 * 292
     assert kernels().count("k_mx_defect") == 1 and sizes == [-(-cells // 256)] * 3, (kernels(), sizes)
     """)
+
+
+def test_layer_grids(host):
+    """Workgroups of the layers that move bytes follow the groups of channels,
+    whatever the shape."""
+    host("""
+    def grid(name, call):
+        got = []
+        answer[name] = lambda stream, size, args: got.append(size) or 0
+        call()
+        return got[0]
+    for n, d, h, w in ((8, 32, 32, 32), (1, 50000, 1, 1), (64, 2, 2, 2)):
+        for c, v in ((16, 8), (20, 1), (3, 1)):
+            assert grid("k_pool_fwd", lambda: nn.pool_fwd(A, A, (n, d, h, w), c)) == -(-n * d * h * w * c // v // 256)
+    assert grid("k_chan_copy", lambda: nn.chan_copy(A, A, 1 << 21, 64, 76, 4, 140, 0, 0)) == 65536
+    """)

@@ -827,14 +827,16 @@ __global__ void k_bf16_to_f32(const bf16_t *__restrict__ a, float *__restrict__ 
 // The layers below move bytes and compute almost nothing: bound is memory, and
 // one 2-byte channel per thread with 64-bit index divisions kept them at 1 to
 // 2 TB/s.  They take V channels per thread (16-byte loads and stores; V = 1
-// for channel counts or addresses that do not allow it), and a workgroup is
-// laid out as V-channel groups by columns by rows, so that the only division
-// is a 32-bit one of the thread index.  Before and now, us: 8 samples of 64^3
-// with 16 channels k_relu_bwd 95 -> 46, k_bias_grad 48 -> 13, k_head_fwd
-// 64 -> 14, k_head_bwd 97 -> 47; a training step of 8 samples of 64^3,
-// both levels: k_up_fwd 363 -> 72, k_pool_bwd 147 -> 60, k_chan_copy
-// 202 -> 133, k_pool_fwd 36 -> 18 (k_up_bwd stays at 101 to 111, bound by
-// the strided gather of its eight children).
+// for channel counts or addresses that do not allow it) and count groups of
+// V channels in 32 bits where those suffice.  Before and now, us: 8 samples of
+// 64^3 with 16 channels k_relu_bwd 95 -> 46, k_bias_grad 48 -> 13, k_head_fwd
+// 64 -> 14, k_head_bwd 97 -> 47; 8 samples of 32^3 (the smaller side)
+// k_pool_fwd 16 channels 26 -> 13, 20 channels (V = 1) 32 -> 21, k_pool_bwd 16
+// channels 103 -> 42, k_up_fwd 64 channels 509 -> 116, k_up_bwd stays at 31
+// (16 channels) and 122 (64), bound by the strided gather of its eight
+// children.  A workgroup laid out as groups by columns by rows of one plane
+// instead: level on those, but 20 channels 51, 50000 planes of one position
+// 34 where this takes 4.
 template <typename T, int V> struct Pack { T v[V]; };
 
 template <typename T, int V>
@@ -854,21 +856,23 @@ __device__ __forceinline__ void store_pack(T *p, const Pack<T, V> &a)
     else *reinterpret_cast<u32x4 *>(p) = __builtin_bit_cast(u32x4, a);
 }
 
-// A workgroup as gc channel groups x gx columns x gy rows of threads.
-struct Lay { int gc, gx, gy; };
-
 // f(plane, y, x, c) for every row y < H, column x < W and first channel c of
-// a group (CV groups of V) of the planes of the launch.
-template <int V, typename F>
-__device__ __forceinline__ void each_group(long long planes, int H, int W, int CV, Lay l, F f)
+// a group (CV groups of V) of `planes` planes.
+template <int V, typename I, typename F>
+__device__ __forceinline__ void each_group_in(I n, int H, int W, int CV, F f)
 {
-    const unsigned t = threadIdx.x, tx = t / (unsigned)l.gc;
-    const int c0 = (int)(t - tx * l.gc), y0 = (int)(tx / (unsigned)l.gx), x0 = (int)(tx - (unsigned)y0 * l.gx);
-    if (y0 >= l.gy) return;
-    for (long long pl = blockIdx.z; pl < planes; pl += gridDim.z)
-        for (long long y = (long long)blockIdx.y * l.gy + y0; y < H; y += (long long)gridDim.y * l.gy)
-            for (long long x = (long long)blockIdx.x * l.gx + x0; x < W; x += (long long)gridDim.x * l.gx)
-                for (int c = c0; c < CV; c += l.gc) f(pl, (int)y, (int)x, c * V);
+    for (I t = (I)blockIdx.x * 256 + threadIdx.x; t < n; t += (I)gridDim.x * 256) {
+        const I p = t / (I)CV, row = p / (I)W, pl = row / (I)H;
+        f((long long)pl, (int)(row - pl * (I)H), (int)(p - row * (I)W), (int)(t - p * (I)CV) * V);
+    }
+}
+
+template <int V, typename F>
+__device__ __forceinline__ void each_group(long long planes, int H, int W, int CV, F f)
+{
+    const long long n = planes * H * W * CV;
+    if (n < (1LL << 31)) each_group_in<V, unsigned>((unsigned)n, H, W, CV, f);
+    else each_group_in<V, long long>(n, H, W, CV, f);
 }
 
 // g_out(bf16) = g(f32) * (y > 0)   (ReLU backward, y = the layer's BF16 output)
@@ -943,9 +947,9 @@ __global__ __launch_bounds__(kBgThreads) void k_bias_grad(const bf16_t *__restri
 // 2x2x2 average pool, channels-last.  in [N][2D][2H][2W][C] -> out [N][D][H][W][C]
 template <int V>
 __global__ __launch_bounds__(256) void k_pool_fwd(const bf16_t *__restrict__ in, bf16_t *__restrict__ out, int N, int D,
-                                                  int H, int W, int C, Lay l)
+                                                  int H, int W, int C)
 {
-    each_group<V>((long long)N * D, H, W, C / V, l, [&](long long zb, int y, int x, int c) {
+    each_group<V>((long long)N * D, H, W, C / V, [&](long long zb, int y, int x, int c) {
         float s[V];
 #pragma unroll
         for (int i = 0; i < V; ++i) s[i] = 0.f;
@@ -966,9 +970,9 @@ __global__ __launch_bounds__(256) void k_pool_fwd(const bf16_t *__restrict__ in,
 // backward of the pool: gin (f32, [N][2D][2H][2W][C]) = gout / 8 (accumulate)
 template <int V>
 __global__ __launch_bounds__(256) void k_pool_bwd(const float *__restrict__ gout, float *__restrict__ gin, int N, int D,
-                                                  int H, int W, int C, Lay l)
+                                                  int H, int W, int C)
 {
-    each_group<V>((long long)N * 2 * D, 2 * H, 2 * W, C / V, l, [&](long long zb, int y, int x, int c) {
+    each_group<V>((long long)N * 2 * D, 2 * H, 2 * W, C / V, [&](long long zb, int y, int x, int c) {
         const Pack<float, V> b = load_pack<float, V>(gout + (((zb >> 1) * H + y / 2) * W + x / 2) * C + c);
         float *p = gin + ((zb * 2 * H + y) * 2 * W + x) * C + c;
         Pack<float, V> a = load_pack<float, V>(p);
@@ -982,9 +986,9 @@ __global__ __launch_bounds__(256) void k_pool_bwd(const float *__restrict__ gout
 // out[N][2D][2H][2W][Ct]; in [N][D][H][W][C]
 template <int V>
 __global__ __launch_bounds__(256) void k_up_fwd(const bf16_t *__restrict__ in, bf16_t *__restrict__ out, int N, int D,
-                                                int H, int W, int C, int Ct, int c0, Lay l)
+                                                int H, int W, int C, int Ct, int c0)
 {
-    each_group<V>((long long)N * 2 * D, 2 * H, 2 * W, C / V, l, [&](long long zb, int y, int x, int c) {
+    each_group<V>((long long)N * 2 * D, 2 * H, 2 * W, C / V, [&](long long zb, int y, int x, int c) {
         const Pack<bf16_t, V> a = load_pack<bf16_t, V>(in + (((zb >> 1) * H + y / 2) * W + x / 2) * C + c);
         store_pack<bf16_t, V>(out + ((zb * 2 * H + y) * 2 * W + x) * Ct + c0 + c, a);
     });
@@ -994,9 +998,9 @@ __global__ __launch_bounds__(256) void k_up_fwd(const bf16_t *__restrict__ in, b
 // channel c0+c in gout[N][2D][2H][2W][Ct]
 template <int V>
 __global__ __launch_bounds__(256) void k_up_bwd(const float *__restrict__ gout, float *__restrict__ gin, int N, int D,
-                                                int H, int W, int C, int Ct, int c0, Lay l)
+                                                int H, int W, int C, int Ct, int c0)
 {
-    each_group<V>((long long)N * D, H, W, C / V, l, [&](long long zb, int y, int x, int c) {
+    each_group<V>((long long)N * D, H, W, C / V, [&](long long zb, int y, int x, int c) {
         Pack<float, V> s;
 #pragma unroll
         for (int i = 0; i < V; ++i) s.v[i] = 0.f;
@@ -1012,29 +1016,23 @@ __global__ __launch_bounds__(256) void k_up_bwd(const float *__restrict__ gout, 
 }
 
 // copy channels: dst[p][dc0 + c] = src[p][sc0 + c], c < C  (concat forward,
-// gradient split backward); T is bf16_t or float.  Positions are the planes
-// of one row of one column, 256 / groups of them per workgroup.
+// gradient split backward); T is bf16_t or float
 template <typename T, int V>
 __global__ __launch_bounds__(256) void k_chan_copy(const T *__restrict__ src, T *__restrict__ dst, long long P, int C,
-                                                   int Cs, int sc0, int Cd, int dc0, int accumulate, Lay l)
+                                                   int Cs, int sc0, int Cd, int dc0, int accumulate)
 {
-    const int CV = C / V;
-    const unsigned po = threadIdx.x / (unsigned)l.gc;
-    const int g0 = (int)(threadIdx.x - po * l.gc);
-    if ((int)po >= l.gx) return;
-    for (long long p = (long long)blockIdx.x * l.gx + po; p < P; p += (long long)gridDim.x * l.gx)
-        for (int c = g0; c < CV; c += l.gc) {
-            Pack<T, V> a = load_pack<T, V>(src + p * Cs + sc0 + c * V);
-            T *d = dst + p * Cd + dc0 + c * V;
-            if constexpr (sizeof(T) == 4) {
-                if (accumulate) {
-                    const Pack<T, V> b = load_pack<T, V>(d);
+    each_group<V>(P, 1, 1, C / V, [&](long long p, int, int, int c) {
+        Pack<T, V> a = load_pack<T, V>(src + p * Cs + sc0 + c);
+        T *d = dst + p * Cd + dc0 + c;
+        if constexpr (sizeof(T) == 4) {
+            if (accumulate) {
+                const Pack<T, V> b = load_pack<T, V>(d);
 #pragma unroll
-                    for (int i = 0; i < V; ++i) a.v[i] = b.v[i] + a.v[i];
-                }
+                for (int i = 0; i < V; ++i) a.v[i] = b.v[i] + a.v[i];
             }
-            store_pack<T, V>(d, a);
         }
+        store_pack<T, V>(d, a);
+    });
 }
 
 // 1x1 head: y[p] = b + sum_c w[c] * x[p][c]   (x BF16, w/b/y FP32)
@@ -1306,22 +1304,10 @@ static bool on16(const void *a, const void *b = nullptr, const void *c = nullptr
     return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) == 0;
 }
 
-// The workgroup of each_group for rows of W columns of groups channel groups,
-// and its grid over H rows of `planes` planes.
-static Lay lay_of(int groups, int W, int H)
+// Workgroups of each_group over n groups of channels.
+static dim3 group_grid(long long n)
 {
-    Lay l;
-    l.gc = std::max(1, std::min(groups, 256));
-    l.gx = std::max(1, std::min(W, 256 / l.gc));
-    l.gy = std::max(1, std::min(H, 256 / (l.gc * l.gx)));
-    return l;
-}
-
-static dim3 lay_grid(const Lay &l, int W, int H, long long planes)
-{
-    auto blocks = [](long long n, long long most) { return (unsigned)std::max(1LL, std::min(n, most)); };
-    return dim3(blocks(((long long)W + l.gx - 1) / l.gx, 1 << 20), blocks(((long long)H + l.gy - 1) / l.gy, 65535),
-                blocks(planes, 65535));
+    return dim3((unsigned)std::max(1LL, std::min((n + 255) / 256, 65536LL)));
 }
 
 static ConvGeom make_conv(int N, int D, int H, int W, int Ci, int Co, int Kpad)
@@ -1607,10 +1593,9 @@ st_status st_nn_pool_fwd(const void *in, void *out, int N, int D, int H, int W, 
     const bf16_t *ib = static_cast<const bf16_t *>(in);
     bf16_t *ob = static_cast<bf16_t *>(out);
     const bool wide = C % 8 == 0 && on16(in, out);
-    const Lay l = lay_of(wide ? C / 8 : C, W, H);
-    const dim3 grid = lay_grid(l, W, H, (long long)N * D);
-    if (wide) hipLaunchKernelGGL(k_pool_fwd<8>, grid, dim3(256), 0, s, ib, ob, N, D, H, W, C, l);
-    else hipLaunchKernelGGL(k_pool_fwd<1>, grid, dim3(256), 0, s, ib, ob, N, D, H, W, C, l);
+    const dim3 grid = group_grid((long long)N * D * H * W * (wide ? C / 8 : C));
+    if (wide) hipLaunchKernelGGL(k_pool_fwd<8>, grid, dim3(256), 0, s, ib, ob, N, D, H, W, C);
+    else hipLaunchKernelGGL(k_pool_fwd<1>, grid, dim3(256), 0, s, ib, ob, N, D, H, W, C);
     return hip_check(hipGetLastError(), "pool launch");
 }
 
@@ -1618,10 +1603,9 @@ st_status st_nn_pool_bwd(const float *gout, float *gin, int N, int D, int H, int
 {
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool wide = C % 4 == 0 && on16(gout, gin);
-    const Lay l = lay_of(wide ? C / 4 : C, 2 * W, 2 * H);
-    const dim3 grid = lay_grid(l, 2 * W, 2 * H, 2LL * N * D);
-    if (wide) hipLaunchKernelGGL(k_pool_bwd<4>, grid, dim3(256), 0, s, gout, gin, N, D, H, W, C, l);
-    else hipLaunchKernelGGL(k_pool_bwd<1>, grid, dim3(256), 0, s, gout, gin, N, D, H, W, C, l);
+    const dim3 grid = group_grid(8LL * N * D * H * W * (wide ? C / 4 : C));
+    if (wide) hipLaunchKernelGGL(k_pool_bwd<4>, grid, dim3(256), 0, s, gout, gin, N, D, H, W, C);
+    else hipLaunchKernelGGL(k_pool_bwd<1>, grid, dim3(256), 0, s, gout, gin, N, D, H, W, C);
     return hip_check(hipGetLastError(), "pool bwd launch");
 }
 
@@ -1632,10 +1616,9 @@ st_status st_nn_up_fwd(const void *in, void *out, int N, int D, int H, int W, in
     const bf16_t *ib = static_cast<const bf16_t *>(in);
     bf16_t *ob = static_cast<bf16_t *>(out);
     const bool wide = (C | Ct | c0) % 8 == 0 && on16(in, out);
-    const Lay l = lay_of(wide ? C / 8 : C, 2 * W, 2 * H);
-    const dim3 grid = lay_grid(l, 2 * W, 2 * H, 2LL * N * D);
-    if (wide) hipLaunchKernelGGL(k_up_fwd<8>, grid, dim3(256), 0, s, ib, ob, N, D, H, W, C, Ct, c0, l);
-    else hipLaunchKernelGGL(k_up_fwd<1>, grid, dim3(256), 0, s, ib, ob, N, D, H, W, C, Ct, c0, l);
+    const dim3 grid = group_grid(8LL * N * D * H * W * (wide ? C / 8 : C));
+    if (wide) hipLaunchKernelGGL(k_up_fwd<8>, grid, dim3(256), 0, s, ib, ob, N, D, H, W, C, Ct, c0);
+    else hipLaunchKernelGGL(k_up_fwd<1>, grid, dim3(256), 0, s, ib, ob, N, D, H, W, C, Ct, c0);
     return hip_check(hipGetLastError(), "upsample launch");
 }
 
@@ -1644,10 +1627,9 @@ st_status st_nn_up_bwd(const float *gout, float *gin, int N, int D, int H, int W
 {
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool wide = (C | Ct | c0) % 4 == 0 && on16(gout, gin);
-    const Lay l = lay_of(wide ? C / 4 : C, W, H);
-    const dim3 grid = lay_grid(l, W, H, (long long)N * D);
-    if (wide) hipLaunchKernelGGL(k_up_bwd<4>, grid, dim3(256), 0, s, gout, gin, N, D, H, W, C, Ct, c0, l);
-    else hipLaunchKernelGGL(k_up_bwd<1>, grid, dim3(256), 0, s, gout, gin, N, D, H, W, C, Ct, c0, l);
+    const dim3 grid = group_grid((long long)N * D * H * W * (wide ? C / 4 : C));
+    if (wide) hipLaunchKernelGGL(k_up_bwd<4>, grid, dim3(256), 0, s, gout, gin, N, D, H, W, C, Ct, c0);
+    else hipLaunchKernelGGL(k_up_bwd<1>, grid, dim3(256), 0, s, gout, gin, N, D, H, W, C, Ct, c0);
     return hip_check(hipGetLastError(), "upsample bwd launch");
 }
 
@@ -1656,10 +1638,8 @@ template <typename T, int V>
 static void chan_copy(const void *src, void *dst, long long P, int C, int Cs, int sc0, int Cd, int dc0, int accumulate,
                       hipStream_t s)
 {
-    Lay l = lay_of(C / V, 256, 1);
-    const unsigned blocks = (unsigned)std::max(1LL, std::min((P + l.gx - 1) / l.gx, 1LL << 20));
-    hipLaunchKernelGGL((k_chan_copy<T, V>), dim3(blocks), dim3(256), 0, s, static_cast<const T *>(src), static_cast<T *>(dst),
-                       P, C, Cs, sc0, Cd, dc0, accumulate, l);
+    hipLaunchKernelGGL((k_chan_copy<T, V>), group_grid(P * (C / V)), dim3(256), 0, s, static_cast<const T *>(src),
+                       static_cast<T *>(dst), P, C, Cs, sc0, Cd, dc0, accumulate);
 }
 }
 
