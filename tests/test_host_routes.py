@@ -104,7 +104,7 @@ def test_mixed_small_kernels(host):
 
 def test_layer_grids(host):
     """Workgroups of the layers that move bytes follow the groups of channels,
-    whatever the shape."""
+    whatever the shape; a loss over many values takes more blocks."""
     host("""
     def grid(name, call):
         got = []
@@ -115,4 +115,6 @@ def test_layer_grids(host):
         for c, v in ((16, 8), (20, 1), (3, 1)):
             assert grid("k_pool_fwd", lambda: nn.pool_fwd(A, A, (n, d, h, w), c)) == -(-n * d * h * w * c // v // 256)
     assert grid("k_chan_copy", lambda: nn.chan_copy(A, A, 1 << 21, 64, 76, 4, 140, 0, 0)) == 65536
+    assert grid("k_sumsq", lambda: nn.sumsq(A, A, A, 1 << 21, 1.0)) == 512
+    assert grid("k_sumsq", lambda: nn.sumsq(A, A, A, 1 << 25, 1.0)) == 2048
     """)

@@ -1310,6 +1310,12 @@ static dim3 group_grid(long long n)
     return dim3((unsigned)std::max(1LL, std::min((n + 255) / 256, 65536LL)));
 }
 
+// Blocks of a sum over n values that ends in one atomic per block on one word,
+// about 13 ns each in turn: 512 up to 2^22 values (2^21 53 us with 4096, 13
+// with 512), then more for the memory's sake, up to 2048 (2^25 102 us with 512,
+// 64 with 2048).
+static long long loss_blocks(long long n) { return std::max(512LL, std::min(n >> 13, 2048LL)); }
+
 static ConvGeom make_conv(int N, int D, int H, int W, int Ci, int Co, int Kpad)
 {
     ConvGeom g;
@@ -1685,7 +1691,7 @@ st_status st_nn_mse(const float *base, const float *y, const float *target, floa
 {
     long long P = (long long)N * n * n * n;
     long long blocks = (P + 255) / 256;
-    if (blocks > 512) blocks = 512;  // one serial atomic per block (8 samples of 64^3: 4096 blocks 56 us, now 32)
+    blocks = std::min(blocks, loss_blocks(P));
     hipLaunchKernelGGL(k_mse, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream), base,
                        y, target, g, loss, pred, N, n, scale);
     return hip_check(hipGetLastError(), "mse launch");
@@ -1711,7 +1717,7 @@ st_status st_nn_axpby(float *out, float a, const float *x, float b, const float 
 st_status st_nn_sumsq(const float *x, float *g, double *loss, long long n, double scale, void *stream)
 {
     long long blocks = (n + 255) / 256;
-    if (blocks > 512) blocks = 512;  // as above (54 -> 15 us)
+    blocks = std::min(blocks, loss_blocks(n));
     hipLaunchKernelGGL(k_sumsq, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream), x,
                        g, loss, n, scale);
     return hip_check(hipGetLastError(), "sumsq launch");
