@@ -118,3 +118,48 @@ def test_layer_grids(host):
     assert grid("k_sumsq", lambda: nn.sumsq(A, A, A, 1 << 21, 1.0)) == 512
     assert grid("k_sumsq", lambda: nn.sumsq(A, A, A, 1 << 25, 1.0)) == 2048
     """)
+
+
+def test_roll_plan(host):
+    """The rolling form's chunks are the best of every chunk count, found
+    without trying them all."""
+    host("""
+    import ctypes, math, random
+    def exhaustive(nx, ny, r, es, steps):
+        cx = 16 // es; ln = 64 * cx; h = (r * steps + cx - 1) // cx * cx
+        nseg = 1 if nx <= ln else -(-(nx - ln) // (ln - 2 * h)) + 1
+        occ = min(8, 512 // (8 * r * steps + (84 if es == 8 else 72)))
+        share = lambda k: (0.0, 1.7, 2.26)[k] if k < 3 else float(k)
+        best = None
+        for nch in range(1, ny + 1):
+            rows = -(-ny // nch)
+            if nch > 1 and rows < 8: break
+            waves = nseg * -(-ny // rows); per = -(-waves // 1024)
+            cost = (per // occ * share(occ) + share(per % occ)) * (rows + 2 * steps * r)
+            if best is None or cost < best[0]: best = (cost, rows, waves)
+        return best[1:]
+    rng = random.Random(7)
+    got = []
+    answer["k_roll"] = lambda stream, size, args: got.append(tuple(ctypes.cast(args[2], ctypes.POINTER(ctypes.c_int))[3:5])) or 0
+    shapes = [(8192, 8192, 4, 0), (19, 60001, 2, 0), (4099, 259, 7, 0), (2051, 2053, 16, 1)]
+    for _ in range(40):
+        nx = int(2 ** rng.uniform(5, 13)); shapes.append((nx, int(2 ** 22.1 / nx * rng.uniform(1, 8)), rng.randint(2, 12), rng.randint(0, 1)))
+    taken = 0
+    for nx, ny, r, f64 in shapes:
+        if min(nx, ny) <= 2 * r: continue
+        p = auto(nx, ny, radius=r, dtype=st.F64 if f64 else st.F32, iterations=4)
+        got.clear()
+        try: st.dispatch_kernels(p, A, B)
+        except st.StencilError: continue  # beyond the launch limits of the family that AUTO names
+        if not got: continue
+        taken += 1
+        steps = st.launch_config(p)["temporal_steps"]
+        rows, waves = exhaustive(nx, ny, r, 8 if f64 else 4, steps)
+        assert got[0] == (waves, rows), (nx, ny, r, f64, got[0], (waves, rows))
+    assert taken > 25
+    p = auto(5, 20000000, radius=2, iterations=4)
+    best = 1e9
+    for _ in range(5):
+        t0 = time.perf_counter(); st.dispatch_kernels(p, A, B); best = min(best, time.perf_counter() - t0)
+    assert best < 2e-3, best
+    """)

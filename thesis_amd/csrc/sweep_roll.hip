@@ -244,10 +244,18 @@ static RollArgs roll_args(const Cfg &c, int steps)
     // 1 / 2 / 3 waves: 129 / 84 / 69 us a sweep).
     const int occ = std::min(8, 512 / (8 * c.r * steps + (es == 8 ? 84 : 72)));
     auto share = [](int k) { return k == 0 ? 0.0 : k == 1 ? 1.7 : k == 2 ? 2.26 : (double)k; };
+    // For k rounds of 1024 waves the best is the most chunks that fit them (the
+    // fewest rows each), so only those are looked at; k rounds cost at least
+    // `least`, the rows of all waves and their halo at the cheapest share, so
+    // the search ends after some ten of them (every chunk count took 20 ms of
+    // host time for 5 x 20000000).
+    const int most = std::max(1, (c.ny - 1) / 7);  // chunks of 8 rows and more
+    const double cheap = share(occ) / occ;
     double best = -1;
-    for (int nch = 1; nch <= c.ny; ++nch) {
-        const int rows = (c.ny + nch - 1) / nch;
-        if (nch > 1 && rows < 8) break;
+    for (long long k = (a.nseg + 1023) / 1024;; ++k) {
+        const double least = cheap * ((double)a.nseg * c.ny / 1024 + (double)k * 2 * steps * c.r);
+        if (best >= 0 && least > best * (1 + 1e-9)) break;
+        const int nch = (int)std::min<long long>(most, 1024 * k / a.nseg), rows = (c.ny + nch - 1) / nch;
         const long long waves = (long long)a.nseg * ((c.ny + rows - 1) / rows), per = (waves + 1023) / 1024;
         const double cost = ((double)(per / occ) * share(occ) + share((int)(per % occ))) * (rows + 2 * steps * c.r);
         if (best < 0 || cost < best) {
@@ -255,6 +263,7 @@ static RollArgs roll_args(const Cfg &c, int steps)
             a.chunk = rows;
             a.nwaves = (int)waves;
         }
+        if (nch == most) break;
     }
     return a;
 }
