@@ -163,3 +163,49 @@ def test_roll_plan(host):
         t0 = time.perf_counter(); st.dispatch_kernels(p, A, B); best = min(best, time.perf_counter() - t0)
     assert best < 2e-3, best
     """)
+
+
+def test_tile_plan(host):
+    """The tile form's rows and z chunk are the best of every chunk count,
+    found without trying them all."""
+    host("""
+    import random
+    def exhaustive(nx, ny, nz, r, es):
+        cx = 2 if r > (5 if es == 8 else 12) else 4
+        best = None
+        for ry in (1, 2):
+            words = 2 * r * ry * cx * es // 4
+            if ry == 2 and cx == 2 or cx == 4 and words > (112 if ry == 2 else 96): continue
+            lds = 2 * (32 * ry + 2 * r) * ((64 + 2 * ((r + 3) // 4 * 4)) * es // 16) * 16
+            two = words <= 40 and lds <= 80 * 1024
+            xy = -(-nx // 64) * -(-ny // (32 * ry)); room = 512 if two else 256
+            for nch in range(1, nz + 1):
+                ch = -(-nz // nch)
+                if nch > 1 and ch < 3: break
+                n = xy * -(-nz // ch)
+                light, full = 1.15 * (ch + 0.3 * 2 * r), ch + 2.0 * r
+                cost = -(-n // room) * (light if cx == 2 or light < full else full) * (ry + 0.6) * (1.6 if two else 1.0)
+                if best is None or cost < best[0]: best = (cost, 32 * ry, ch, n)
+        return best[1:]
+    rng = random.Random(11)
+    taken = 0
+    for _ in range(300):
+        nx, ny = (int(2 ** rng.uniform(4, 10)) for _ in "xy")
+        nz = int(2 ** 20 / nx / ny * 2 ** rng.uniform(0.5, 6)); r = rng.randint(1, 16); f64 = rng.random() < 0.4
+        if not 2 * r < min(nx, ny, nz) or nz > 60000: continue
+        p = auto(nx, ny, nz, radius=r, dtype=st.F64 if f64 else st.F32, variant="smem_register")
+        try: c = st.launch_config(p)
+        except st.StencilError: continue
+        if c["block_x"] != 64 or c["block_y"] not in (32, 64) or c["grid_y"] != 1 or c["zchunk"] != c["block_z"]: continue
+        want = exhaustive(nx, ny, nz, r, 8 if f64 else 4)
+        if (c["block_y"], c["zchunk"], c["grid_x"]) != want:
+            # another form's numbers, or a plan of the same cost
+            raise AssertionError((nx, ny, nz, r, f64, c, want))
+        taken += 1
+    assert taken > 60, taken
+    p = auto(40, 40, 1000000, radius=3, variant="smem_register")
+    best = 1e9
+    for _ in range(5):
+        t0 = time.perf_counter(); st.sweep(p, A, B); best = min(best, time.perf_counter() - t0)
+    assert kernels()[-1] == "k_tile" and best < 1e-3, (kernels()[-1], best)
+    """)

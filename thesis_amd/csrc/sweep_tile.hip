@@ -411,11 +411,19 @@ st_status resolve_tile(Cfg &c)
         if (!t.fn) continue;
         const int per_cu = t.words <= 40 && t.lds <= kMaxLds / 2 ? 2 : 1;
         const long long xy = (long long)((c.nx + kTileX - 1) / kTileX) * ((c.ny + 32 * ry - 1) / (32 * ry));
-        for (int nch = 1; nch <= c.nz; ++nch) {
-            const int ch = (c.nz + nch - 1) / nch;
-            if (nch > 1 && ch < 3) break;
+        // For k rounds the most chunks that fit them are the best, and k
+        // rounds take at least the planes of all chunks and their halo: the
+        // search ends after some ten of them (every chunk count took 0.3 ms
+        // of host time for 9 x 9 x 100000).
+        const long long room = (long long)cus * per_cu;
+        const int most = std::max(1, (c.nz - 1) / 2);  // chunks of 3 planes and more
+        const double rows = (ry + 0.6) * (per_cu == 2 ? 1.6 : 1.0);
+        for (long long k = (xy + room - 1) / room;; ++k) {
+            const double least = ((double)xy * c.nz / room + 0.69 * c.r * k) * rows;
+            if (best >= 0 && least > best * (1 + 1e-9)) break;
+            const int nch = (int)std::min<long long>(most, room * k / xy), ch = (c.nz + nch - 1) / nch;
             const long long n = xy * ((c.nz + ch - 1) / ch);
-            const double cost = (double)((n + cus * per_cu - 1) / (cus * per_cu)) * tile_work(c, ch, tile_light(c, ch)) * (ry + 0.6) * (per_cu == 2 ? 1.6 : 1.0);
+            const double cost = (double)((n + room - 1) / room) * tile_work(c, ch, tile_light(c, ch)) * rows;
             if (best < 0 || cost < best) {
                 best = cost;
                 c.cy = ry;
@@ -423,6 +431,7 @@ st_status resolve_tile(Cfg &c)
                 c.lds = t.lds;
                 c.gx = (int)n;
             }
+            if (nch == most) break;
         }
     }
     if (best < 0) return fail(ST_EUNSUPPORTED, "tile form: no kernel for radius %d", c.r);
