@@ -209,3 +209,24 @@ def test_tile_plan(host):
         t0 = time.perf_counter(); st.sweep(p, A, B); best = min(best, time.perf_counter() - t0)
     assert kernels()[-1] == "k_tile" and best < 1e-3, (kernels()[-1], best)
     """)
+
+
+def test_small_interiors(host):
+    """Grids whose interior is a small part of their tiles stay with the kernels
+    they had: the register march or the plain kernel."""
+    host("""
+    def route(nx, ny, nz, r, dt=st.F32):
+        log.clear()
+        st.dispatch_kernels(auto(nx, ny, nz, radius=r, dtype=dt, iterations=2), A, B)
+        return kernels()[-1]
+    march = {(1000, 33, 33): (6, 8), (4000, 20, 20): (6, 8), (40, 4000, 20): (8,), (9, 9, 100000): (1,)}
+    plain = {(1000, 33, 33): (10, 12), (104, 104, 104): (10, 12), (33, 33, 2000): (12,), (33, 33, 5000): (16,)}
+    plain64 = {(1000, 33, 33): (5, 6, 8), (4000, 20, 20): (5, 6, 8), (33, 33, 2000): (10,), (12000, 12000, 11): (5,)}
+    tile = {(1000, 33, 33): (2, 4), (1000, 1000, 20): (6, 8), (2000, 500, 24): (10,), (104, 104, 104): (6, 8), (64, 64, 400): (12,),
+            (128, 128, 128): (6, 8, 10, 12), (333, 251, 207): (1, 2, 6, 12, 16), (20, 20, 40000): (2, 8)}
+    tile64 = {(128, 128, 128): (3, 5, 8, 10), (104, 104, 104): (5, 6, 8), (40, 4000, 20): (6, 8), (2000, 500, 24): (10,)}
+    for want, dt, cases in (("k_march", st.F32, march), ("k_base", st.F32, plain), ("k_base", st.F64, plain64),
+                            ("k_tile", st.F32, tile), ("k_tile", st.F64, tile64), ("k_rowc", st.F64, {(256, 256, 256): (3,)})):
+        for shape, radii in cases.items():
+            for r in radii: assert route(*shape, r, dt).startswith(want), (shape, r, dt, route(*shape, r, dt))
+    """)

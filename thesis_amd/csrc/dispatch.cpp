@@ -244,13 +244,15 @@ static st_status resolve(const st_params *p, Cfg &c, bool mixed)
             c.variant = ST_V_BASE;
             c.cx = 1;
         } else {
-            // 3D: FP32 up to radius 14, FP64 up to 8, and where the tile form
-            // is ahead (us per sweep, plain / this: FP32 320x256x256 R=14
-            // 602 / 311, 384^3 R=16 805 / 301; FP64 192^3 R=3 86 / 25, R=9
-            // 138 / 75; the register march of radius 16 is behind, 394 / 1206)
-            const bool march_ok = c.dims == 3 ? c.r <= (c.dtype == ST_F64 ? 8 : 14) || tile_eligible(c)
-                                              : (c.dtype == ST_F32 && c.r <= 8) ||
-                                                    (c.dtype == ST_F64 && (c.r == 1 || c.r == 2 || c.r == 4));
+            // the register march's radii, and in 3D where the tile form is
+            // ahead of the plain kernel (us per sweep, plain / this: FP32
+            // 320x256x256 R=14 602 / 311, 384^3 R=16 805 / 301; FP64 192^3 R=3
+            // 86 / 25, R=9 138 / 75) or the row form serves radius 3 in FP64
+            // (256^3 198 / 48)
+            const bool march_ok = (c.dtype == ST_F32 && c.r <= 8) ||
+                                  (c.dtype == ST_F64 && (c.r == 1 || c.r == 2 || c.r == 4)) ||
+                                  (c.dims == 3 && ((c.r <= 4 && rows_consecutive(c)) ||
+                                                   (tile_eligible(c) && tile_over_plain(c))));
             c.variant = march_ok ? ST_V_SMEM_REGISTER : ST_V_BASE;
             if (!march_ok) c.cx = 1;
         }

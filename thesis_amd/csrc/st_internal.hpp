@@ -75,8 +75,10 @@ st_status run_rows_coop(const Cfg &c, void *u1, void *u2, hipStream_t s, int *in
 st_status launch_rows(const Cfg &c, const void *in, void *out, hipStream_t s);
 bool rows_consecutive(const Cfg &c);  // the row form would take its consecutive layout
 // SMEM_REGISTER tile form, one sweep (sweep_tile.hip); eligible: the
-// library's choice for the shape.
+// library's choice for the shape among the SMEM_REGISTER forms; over_plain:
+// AUTO's choice between it and the plain kernel.
 bool tile_eligible(const Cfg &c);
+bool tile_over_plain(const Cfg &c);
 st_status resolve_tile(Cfg &c);
 st_status launch_tile(const Cfg &c, const void *in, void *out, hipStream_t s);
 // 16-bit storage modes on the geometry of `c` (FP32 arithmetic, JACOBI

@@ -382,6 +382,22 @@ static bool tile_light(const Cfg &c, int ch) { return tile_cx(c) == 2 || tile_wo
 //   * else the tile is ahead: 320^3 FP32 R = 2 59 / 54, R = 4 75 / 61; widths
 //     that are no multiple of 4, which only the register march took, 1.25x
 //     (R = 1) to 4.3x (R = 4).
+//   * a tile computes shell cells like any other and marches through 2R planes
+//     of halo: FP32 radii 6 to 8 stay with the register march where little of
+//     the grid is interior (1000x33x33 R = 8 11 / 16.5, R = 6 10.9 / 14), up to
+//     a larger size where that has fewer planes than the halo (40x4000x20
+//     R = 8 10 / 12.6, 1000x1000x20 R = 6 40 / 25.5), and radius 1 where 15/16 of
+//     the tiles lie outside (9x9x100000 93 / 118).
+static long long ceil_to(long long n, long long unit) { return (n + unit - 1) / unit * unit; }
+
+// Interior cells, rows rounded up to the 64 lanes of a wave; cells of the
+// tiles, a plane of z halo as 0.3.
+static long long interior_rounded(const Cfg &c)
+{
+    return ceil_to(c.nx - 2 * c.r, 64) * (c.ny - 2 * c.r) * (c.nz - 2 * c.r);
+}
+static long long tiles_rounded(const Cfg &c) { return ceil_to(c.nx, kTileX) * ceil_to(c.ny, 32) * (c.nz - 2 * c.r + 6 * c.r / 10); }
+
 bool tile_eligible(const Cfg &c)
 {
     if (c.dims != 3 || (c.dtype != ST_F32 && c.dtype != ST_F64)) return false;
@@ -392,7 +408,23 @@ bool tile_eligible(const Cfg &c)
     if (((long long)c.nx * (c.ny + 2 * c.r + 64) + 128) * es >= (1LL << 30)) return false;
     if (c.r <= 4 && c.nx % 4 == 0 && (rows_consecutive(c) || (c.nx > 512 && c.r <= (es == 8 ? 2 : 1))))
         return false;
+    if (c.r == 1 && 16 * cells < tiles_rounded(c)) return false;
+    if (es == 4 && c.r >= 6 && c.r <= 8 && interior_rounded(c) < (c.nz < 4 * c.r ? 3LL << 20 : 5LL << 17)) return false;
     return tile_kernel_for(c, 1, tile_cx(c), true).fn != nullptr;
+}
+
+// AUTO's rule between the tile form and the plain kernel, which computes the
+// interior alone (FP32 from radius 9, FP64 radius 3 and from 5; us per sweep,
+// plain / tile): it is ahead while the interior is small (FP32 1000x33x33 R = 10
+// 7 / 19, 104^3 R = 12 18 / 20, 128^3 R = 12 31 / 21; FP64 1000x33x33 R = 8 9.7 /
+// 19.6, 4000x20x20 R = 6 12.6 / 14.3, 104^3 R = 8 29 / 21), and where the slower
+// kernels of wide stars spend themselves on shell cells (33x33x2000 FP64 R = 10
+// 48 / 93, FP32 R = 12 30 / 37; 2000x500x24 FP64 R = 10 148 / 121).
+bool tile_over_plain(const Cfg &c)
+{
+    const long long in = interior_rounded(c), all = tiles_rounded(c);
+    if (c.dtype == ST_F32) return c.r < 9 || (in >= 7LL << 17 && 25 * in >= 4 * all);
+    return c.r < 5 || (c.r < 9 ? in >= 5LL << 17 : 20 * in >= 7 * all);
 }
 
 st_status resolve_tile(Cfg &c)
