@@ -230,3 +230,15 @@ def test_small_interiors(host):
         for shape, radii in cases.items():
             for r in radii: assert route(*shape, r, dt).startswith(want), (shape, r, dt, route(*shape, r, dt))
     """)
+
+
+def test_tile_shell_comparison(host):
+    """A short run in the tile form does not pay for comparing the shells."""
+    host("""
+    def compared(n, r, its):
+        log.clear()
+        st.dispatch_kernels(auto(n, n, n, radius=r, iterations=its), A, B)
+        assert kernels()[-1] == "k_tile"
+        return "k_grid_shell_eq" in kernels()
+    assert not compared(128, 6, 2) and compared(128, 6, 8) and not compared(320, 2, 1) and compared(320, 2, 2)
+    """)

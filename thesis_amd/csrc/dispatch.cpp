@@ -405,9 +405,14 @@ st_status stencil_dispatch(const st_params *p, void *d_u1, void *d_u2, void *str
         } else if (c.variant == ST_V_COOP) {
             s = run_coop(c, d_u1, d_u2, hs, &in_u2);
         } else {
-            // the row form stores whole rows when both shells are equal
-            // (a shell cell then holds the same bits at every sweep)
-            if (c.variant == ST_V_SMEM_REGISTER && (c.kind == 4 || c.kind == 8) && c.iters > 1)
+            // the row and tile forms store whole rows when both shells are
+            // equal (a shell cell then holds the same bits at every sweep).
+            // The comparison's two launches take about 5 us: the tile form,
+            // most of whose words are whole anyway, earns them back over 2^23
+            // cells in all (128^3 R = 6, 2 sweeps, with / without the
+            // comparison: 34 / 26 us; 12x400x400 FP64 R = 1, 7 sweeps: 148 / 164)
+            const bool repaid = (long long)c.iters * c.nx * c.ny * c.nz >= 1LL << 23;
+            if (c.variant == ST_V_SMEM_REGISTER && (c.kind == 4 || (c.kind == 8 && repaid)) && c.iters > 1)
                 s = rows_shell_check(c, d_u1, d_u2, hs, &c.shell_eq);
             void *a = d_u1, *b = d_u2;
             for (int i = 0; i < c.iters && s == ST_OK; ++i) {
