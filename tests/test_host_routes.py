@@ -242,3 +242,19 @@ def test_tile_shell_comparison(host):
         return "k_grid_shell_eq" in kernels()
     assert not compared(128, 6, 2) and compared(128, 6, 8) and not compared(320, 2, 1) and compared(320, 2, 2)
     """)
+
+
+def test_roll_small_planes(host):
+    """Planes that are mostly shell rows, and few sweeps of radius 2 over small
+    planes of whole quads, stay with the kernels they had."""
+    host("""
+    def rolls(nx, ny, r, its=16, dt=st.F32, op=1):
+        log.clear()
+        st.dispatch_kernels(auto(nx, ny, radius=r, dtype=dt, iterations=its, op=op), A, B)
+        return kernels()[-1] == "k_roll"
+    assert not rolls(100000, 40, 16, dt=st.F64) and rolls(100000, 40, 12, dt=st.F64)
+    assert not rolls(300000, 9, 4, dt=st.F64) and rolls(300000, 9, 3, dt=st.F64)
+    assert not rolls(1024, 1024, 2, 7, op=0) and not rolls(1024, 1024, 2, 3) and rolls(1024, 1024, 2, 16)
+    assert rolls(1031, 1021, 2, 4) and rolls(2048, 2048, 2, 3) and not rolls(64, 60000, 2, 7, op=0) and rolls(1024, 1024, 3, 3)
+    assert not rolls(1024, 1024, 2, 3, dt=st.F64) and rolls(1024, 1024, 2, 4, dt=st.F64) and rolls(64, 60000, 2, 3, dt=st.F64)
+    """)

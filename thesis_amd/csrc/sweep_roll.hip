@@ -286,8 +286,22 @@ void resolve_roll(Cfg &c)
     if (c.dims != 2 || (c.dtype != ST_F32 && c.dtype != ST_F64) || c.nx < 2 * c.r + 1 || c.ny < 2 * c.r + 1) return;
     const long long es = c.dtype == ST_F64 ? 8 : 4, cells = (long long)c.nx * c.ny;
     if (cells * es >= (1LL << 31)) return;  // 32-bit byte offsets
+    // a wave marches through the shell's rows too: not where they are over
+    // three quarters (FP64 100000x40 R = 16, 8 rows of 40, 24 / 32; 300000x9
+    // R = 4 5.8 / 6.4)
+    if (4LL * (c.ny - 2 * c.r) < c.ny) return;
     const bool late = c.dtype == ST_F32 && (c.r % 4 == 0 || c.r > 8);
     if (cells < (late ? 1LL << 22 : 1LL << 20) || !roll_kernel(c, 1)) return;
+    // Radius 2 on whole quads, the plain kernel's best case: up to 2^21 cells
+    // (for FP32 not counting columns that a segment of 256 leaves empty) few
+    // sweeps, and FP32 THESIS, stay with it (us, plain / this: 1024^2 3 sweeps
+    // 14.9 / 16.8, FP64 19.1 / 20.6, 7 of THESIS 34.5 / 38.6, 16 of JACOBI 85 / 79;
+    // 64x60000 7 of THESIS 74 / 86).
+    if (c.r == 2 && c.nx % 4 == 0) {
+        const bool f32 = c.dtype == ST_F32;
+        const long long filled = f32 ? cells * std::min(c.nx, 256) / 256 : cells;
+        if (filled < 1LL << 21 && (c.iters < 4 || (f32 && (c.op == OP_THESIS || c.iters < 8)))) return;
+    }
     const bool deep = roll_kernel(c, kRollSteps) && (c.r <= 3 || cells * es >= 32LL << 20 << (c.r - 4));
     c.roll_steps = deep ? kRollSteps : 1;
 }
