@@ -258,3 +258,42 @@ def test_roll_small_planes(host):
     assert rolls(1031, 1021, 2, 4) and rolls(2048, 2048, 2, 3) and not rolls(64, 60000, 2, 7, op=0) and rolls(1024, 1024, 3, 3)
     assert not rolls(1024, 1024, 2, 3, dt=st.F64) and rolls(1024, 1024, 2, 4, dt=st.F64) and rolls(64, 60000, 2, 3, dt=st.F64)
     """)
+
+
+def test_workspace_growth_and_capture(host):
+    """Growing the workspace neither ends a capture on another stream nor takes
+    a block away from a captured graph; a block that cannot be freed is kept."""
+    host("""
+    mode, capturing, freed, blocks = [0], set(), [], []
+    answer["mode"] = lambda h, n, a: mode.__setitem__(0, n) or 0
+    answer["capturing"] = lambda h, n, a: int(h in capturing)
+    def guarded(h, n, a): return 900 if capturing and mode[0] != 2 else 0    # stream capture would be ended
+    def free(h, n, a):
+        if not guarded(h, n, a): freed.append(h)
+        return guarded(h, n, a)
+    answer["malloc"], answer["free"] = guarded, free
+    answer["sync"] = lambda h, n, a: 900 if h in capturing else 0
+    answer["k_pc_transpose"] = lambda h, n, a: blocks.append(C.cast(a[1], C.POINTER(C.c_void_p))[0]) or 0
+    def call(stream, pos):  # 128 + 64 channel-major words of 2 bytes a position in the workspace
+        log.clear(); blocks.clear()
+        nn.conv3_wgrad(A, A, A, (1, 1, 1, pos), 64, 64, stream=stream)
+        assert kernels()[-1] == "k_conv3_wgrad_t"
+        return blocks[0]
+    S, T = 0x5000, 0x6000
+    a = call(S, 1 << 18)
+    capturing.add(T)
+    b = call(S, 1 << 19)                       # grows while T is under capture
+    assert freed == [a] and b != a
+    c = call(T, 1 << 18)                       # first use, under capture
+    d = call(T, 1 << 19)                       # grows under capture: nothing waited for, nothing freed
+    assert freed == [a] and d != c
+    capturing.clear()
+    call(T, 1 << 22)                           # grows outside: c and d belong to the captured graph
+    assert freed == [a]
+    answer["free"] = 1
+    try: call(S, 1 << 22); raise SystemExit("growth without its free")
+    except st.StencilError: pass
+    answer["free"] = free
+    e = call(S, 1 << 22)
+    assert freed == [a, b] and e not in (a, b)
+    """)

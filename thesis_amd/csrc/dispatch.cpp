@@ -8,14 +8,16 @@
 // as status codes; nothing here exits the process.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
 #include <map>
 #include <mutex>
-#include <tuple>
 #include <string>
+#include <tuple>
+#include <vector>
 
 #include "st_internal.hpp"
 
@@ -53,6 +55,8 @@ constexpr int kSlots = 5;
 struct WsBlock {
     void *ptr = nullptr;
     size_t size = 0;
+    bool captured = false;     // a graph recorded by the caller may hold ptr
+    std::vector<void *> idle;  // outgrown under capture, freed by the next growth outside
 };
 static std::map<std::tuple<int, hipStream_t, int>, WsBlock> g_ws;
 
@@ -62,6 +66,13 @@ static thread_local const WsFixed *g_ws_fixed = nullptr;
 
 void workspace_use_fixed(const WsFixed *fixed) { g_ws_fixed = fixed; }
 bool workspace_is_fixed() { return g_ws_fixed != nullptr; }
+
+// Relaxed capture mode of this thread while it lives.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
 
 st_status workspace_slot(int slot, size_t bytes, hipStream_t stream, void **ptr, size_t *fresh)
 {
@@ -81,25 +92,40 @@ st_status workspace_slot(int slot, size_t bytes, hipStream_t stream, void **ptr,
     if (e != hipSuccess) return hip_check(e, "hipGetDevice");
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     WsBlock &w = g_ws[std::make_tuple(dev, stream, slot)];
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) (void)hipGetLastError();
+    const bool capturing = cap != hipStreamCaptureStatusNone;
     if (w.size < bytes) {
-        if (w.ptr) {
-            // earlier work on this stream may still use the old block
-            e = hipStreamSynchronize(stream);
-            if (e != hipSuccess) return hip_check(e, "workspace sync");
-            (void)hipFree(w.ptr);
-            w.ptr = nullptr;
-            w.size = 0;
+        // Another stream of this thread may be under capture: freeing and
+        // allocating here must not end it.
+        RelaxedCapture relaxed;
+        // A block that a captured graph may use stays for its replays, and
+        // under capture nothing can be waited for: such growth at least
+        // doubles, so what stays behind is less than the block in use.
+        size_t sz = std::max<size_t>(bytes, 1u << 20);
+        if (w.captured || capturing) sz = std::max(sz, 2 * w.size);
+        if (!capturing && (w.ptr || !w.idle.empty())) {
+            // earlier work on this stream may still use the old blocks
+            if ((e = hipStreamSynchronize(stream)) != hipSuccess) return hip_check(e, "workspace sync");
+            if (w.ptr && !w.captured) {
+                w.idle.push_back(w.ptr);
+                w.ptr = nullptr;
+                w.size = 0;
+            }
+            while (!w.idle.empty()) {
+                if ((e = hipFree(w.idle.back())) != hipSuccess) return hip_check(e, "workspace hipFree");
+                w.idle.pop_back();
+            }
         }
-        size_t sz = bytes < (1u << 20) ? (1u << 20) : bytes;
-        // another stream of this thread may be under capture
-        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-        (void)hipThreadExchangeStreamCaptureMode(&mode);
-        e = hipMalloc(&w.ptr, sz);
-        (void)hipThreadExchangeStreamCaptureMode(&mode);
-        if (e != hipSuccess) return hip_check(e, "workspace hipMalloc");
+        void *grown = nullptr;
+        if ((e = hipMalloc(&grown, sz)) != hipSuccess) return hip_check(e, "workspace hipMalloc");
+        if (w.ptr && !w.captured) w.idle.push_back(w.ptr);
+        w.ptr = grown;
         w.size = sz;
+        w.captured = false;
         if (fresh) *fresh = sz;
     }
+    w.captured |= capturing;
     *ptr = w.ptr;
     return ST_OK;
 }
