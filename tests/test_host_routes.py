@@ -297,3 +297,37 @@ def test_workspace_growth_and_capture(host):
     e = call(S, 1 << 22)
     assert freed == [a, b] and e not in (a, b)
     """)
+
+
+def test_threads_on_one_stream(host):
+    """Each call's launches on a stream come in one piece, also the first ones,
+    which allocate: what they leave in the stream's workspace is theirs."""
+    host("""
+    def pause(h, n, a): time.sleep(0.0005); return 0
+    for k in ("k_flag_one", "k_grid_shell_eq", "k_tile", "k_resident_clear", "k_resident", "k_conv3_wgrad_tile", "k_wgrad_reduce",
+              "capturing", "malloc", "mode"): answer[k] = pause
+    def calls(stream):
+        for _ in range(3):
+            st.dispatch_kernels(auto(96, 96, 96, iterations=24), A, B, stream=stream)
+            st.dispatch_kernels(auto(200, 200, 100, radius=2, iterations=4), A, B, stream=stream)
+            nn.conv3_wgrad(A, A, A, (8, 16, 16, 16), 16, 16, stream=stream)
+    want = [["k_resident"], ["k_flag_one", "k_grid_shell_eq"] + ["k_tile"] * 4, ["k_conv3_wgrad_tile", "k_wgrad_reduce"]] * 3
+    for stream in (0x5000, 0x6000):
+        log.clear()
+        ts = [threading.Thread(target=calls, args=(stream,)) for _ in range(4)]
+        [t.start() for t in ts]; [t.join() for t in ts]
+        got = [(e[0], e[3]) for e in log if e[0].startswith("k_") and e[0] != "k_resident_clear"]
+        first = [e[0] for e in log if e[0].startswith("k_resident")]
+        assert first[0] == "k_resident_clear" and first.count("k_resident_clear") == 1, first
+        runs = []  # launches of one thread in a row
+        for name, t in got:
+            if runs and runs[-1][1] == t: runs[-1][0].append(name)
+            else: runs.append(([name], t))
+        flat = {}
+        for names, t in runs:
+            seq = flat.setdefault(t, [])
+            seq += names
+            done = [n for w in want for n in w][:len(seq)]
+            ends = [sum(map(len, want[:i])) for i in range(len(want) + 1)]
+            assert seq == done and len(seq) in ends, (names, seq)
+    """)

@@ -49,7 +49,7 @@ st_status hip_check(hipError_t e, const char *what)
 
 // One workspace per (device, stream, slot): calls on different streams never
 // share device scratch (shell flags, reduction partials, batch tables), and
-// calls on one stream are ordered by the stream.
+// calls on one stream are ordered by the stream, each whole (StreamTurn).
 static std::mutex g_ws_mutex;
 constexpr int kSlots = 5;
 struct WsBlock {
@@ -66,6 +66,16 @@ static thread_local const WsFixed *g_ws_fixed = nullptr;
 
 void workspace_use_fixed(const WsFixed *fixed) { g_ws_fixed = fixed; }
 bool workspace_is_fixed() { return g_ws_fixed != nullptr; }
+
+StreamTurn::StreamTurn(hipStream_t stream)
+{
+    // streams that share an entry only wait for each other's launches
+    static std::recursive_mutex turns[64];
+    mutex_ = &turns[(reinterpret_cast<uintptr_t>(stream) >> 4) * 0x9E3779B97F4A7C15ull >> 58];
+    static_cast<std::recursive_mutex *>(mutex_)->lock();
+}
+
+StreamTurn::~StreamTurn() { static_cast<std::recursive_mutex *>(mutex_)->unlock(); }
 
 // Relaxed capture mode of this thread while it lives.
 struct RelaxedCapture {
@@ -415,6 +425,7 @@ st_status stencil_dispatch(const st_params *p, void *d_u1, void *d_u2, void *str
         if ((s = hip_check(hipEventRecord(e0, hs), "event record")) != ST_OK) goto done;
     }
     {
+        StreamTurn turn(hs);
         int in_u2 = 0;
         bool done = false;
         if (c.resident) {
@@ -491,6 +502,7 @@ st_status stencil_residual_norm(const st_params *p, const void *d_u, double *nor
     st_status s = resolve_geometry(p, c);
     if (s != ST_OK) return s;
     if (!d_u || !norm) return fail(ST_EINVAL, "null argument");
+    StreamTurn turn(static_cast<hipStream_t>(stream));
     return residual_norm(c, d_u, norm, static_cast<hipStream_t>(stream));
 }
 
@@ -534,7 +546,11 @@ st_status stencil_dispatch_batched(const st_problem *problems, int nproblems,
         if (s != ST_OK) return s;
         hs = own;
     }
-    st_status s = run_batched(problems, nproblems, rules, nrules, mode, hs, elapsed_ms);
+    st_status s;
+    {
+        StreamTurn turn(hs);
+        s = run_batched(problems, nproblems, rules, nrules, mode, hs, elapsed_ms);
+    }
     if (own) {
         (void)hipStreamSynchronize(own);
         (void)hipStreamDestroy(own);

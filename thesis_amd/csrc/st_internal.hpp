@@ -143,6 +143,20 @@ st_status run_mixed(const Cfg &c, void *x, void *e1, void *e2, void *d, void *u,
 
 // Library-owned device workspace (grows on demand, one per device, stream
 // and slot).
+// A call that uses workspace holds its stream's turn while it enqueues, so
+// that what other threads enqueue on the stream comes before or after all of
+// it (the workspace is the stream's).  Calls within calls may take it again.
+class StreamTurn {
+public:
+    explicit StreamTurn(hipStream_t stream);
+    ~StreamTurn();
+    StreamTurn(const StreamTurn &) = delete;
+    StreamTurn &operator=(const StreamTurn &) = delete;
+
+private:
+    void *mutex_;
+};
+
 // *fresh (optional) receives the block's size when this call allocated it,
 // else 0.
 st_status workspace_slot(int slot, size_t bytes, hipStream_t stream, void **ptr, size_t *fresh = nullptr);

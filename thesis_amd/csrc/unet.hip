@@ -1508,6 +1508,7 @@ st_status st_nn_conv3_wgrad(const void *x, const void *dy, float *dw, int N, int
     const ConvGeom g = make_conv(N, D, H, W, Ci, Co, st_nn_kpad(Ci));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bf16_t *xb = static_cast<const bf16_t *>(x), *yb = static_cast<const bf16_t *>(dy);
+    StreamTurn turn(s);
     const WgradTilePlan t = wgrad_tile_plan(g);
     const WgradForm form = wgrad_form(g, t);
     if (form == WG_TILE) {
