@@ -331,3 +331,20 @@ def test_threads_on_one_stream(host):
             ends = [sum(map(len, want[:i])) for i in range(len(want) + 1)]
             assert seq == done and len(seq) in ends, (names, seq)
     """)
+
+
+def test_per_thread_stream(host):
+    """hipStreamPerThread is another stream on each thread, with a workspace
+    of its own."""
+    host("""
+    blocks = set()
+    answer["k_flag_one"] = lambda h, n, a: blocks.add((threading.get_ident(), C.cast(a[0], C.POINTER(C.c_void_p))[0])) or 0
+    barrier = threading.Barrier(3)
+    def call():
+        barrier.wait()
+        for _ in range(3): st.dispatch_kernels(auto(200, 200, 100, radius=2, iterations=4), A, B, stream=2)
+        barrier.wait()
+    ts = [threading.Thread(target=call) for _ in range(3)]
+    [t.start() for t in ts]; [t.join() for t in ts]
+    assert len(blocks) == 3 and len({b for _, b in blocks}) == 3, blocks
+    """)

@@ -50,6 +50,8 @@ st_status hip_check(hipError_t e, const char *what)
 // One workspace per (device, stream, slot): calls on different streams never
 // share device scratch (shell flags, reduction partials, batch tables), and
 // calls on one stream are ordered by the stream, each whole (StreamTurn).
+// hipStreamPerThread names another stream on every thread, so its blocks
+// belong to the thread too.
 static std::mutex g_ws_mutex;
 constexpr int kSlots = 5;
 struct WsBlock {
@@ -58,7 +60,7 @@ struct WsBlock {
     bool captured = false;     // a graph recorded by the caller may hold ptr
     std::vector<void *> idle;  // outgrown under capture, freed by the next growth outside
 };
-static std::map<std::tuple<int, hipStream_t, int>, WsBlock> g_ws;
+static std::map<std::tuple<int, hipStream_t, const void *, int>, WsBlock> g_ws;
 
 // While set on this thread, workspace requests are served from a fixed
 // device buffer (one part per slot) and nothing is allocated.
@@ -101,7 +103,9 @@ st_status workspace_slot(int slot, size_t bytes, hipStream_t stream, void **ptr,
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_check(e, "hipGetDevice");
     std::lock_guard<std::mutex> lock(g_ws_mutex);
-    WsBlock &w = g_ws[std::make_tuple(dev, stream, slot)];
+    static thread_local char thread_key;
+    const void *owner = stream == hipStreamPerThread ? &thread_key : nullptr;
+    WsBlock &w = g_ws[std::make_tuple(dev, stream, owner, slot)];
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cap) != hipSuccess) (void)hipGetLastError();
     const bool capturing = cap != hipStreamCaptureStatusNone;
