@@ -348,3 +348,22 @@ def test_per_thread_stream(host):
     [t.start() for t in ts]; [t.join() for t in ts]
     assert len(blocks) == 3 and len({b for _, b in blocks}) == 3, blocks
     """)
+
+
+def test_no_room_for_workspace(host):
+    """Calls that ran without a workspace before they were given a faster form
+    still run where there is no room for one."""
+    host("""
+    answer["malloc"] = 2  # hipErrorOutOfMemory
+    def route(call):
+        log.clear(); call()
+        return kernels()
+    run = lambda *a, **kw: st.dispatch_kernels(auto(*a, **kw), A, B)
+    assert route(lambda: run(64, 64, 64, iterations=24))[0].startswith("k_base")
+    assert route(lambda: run(128, 128, 128, iterations=24)) == ["k_tile"] * 24
+    assert route(lambda: run(333, 251, 207, radius=2)) == ["k_tile"] * 4
+    assert route(lambda: nn.conv3_wgrad(A, A, A, (2, 33, 33, 33), 16, 16)) == ["k_conv3_wgrad"]
+    problems = [dict(nx=64, ny=40, nz=33, radius=1, iterations=24, op=1, u1=A, u2=B)] * 4
+    try: st.dispatch_batched(problems, (), st.BATCH_PERSISTENT, stream=0x5000)
+    except st.StencilError as e: assert e.status == 4  # its own table needs memory, as before
+    """)

@@ -477,6 +477,11 @@ st_status run_resident(const Cfg &c, int problems, void *const (*u)[2], hipStrea
     void *ws = nullptr;
     size_t fresh = 0;
     st_status st = workspace_slot(kSlotResident, bytes, s, &ws, &fresh);
+    if (st == ST_ENOMEM) {
+        // no room for the faces: the caller's other form, which needs none
+        (void)hipGetLastError();
+        return ST_OK;
+    }
     if (st != ST_OK) return st;
     if (fresh) {
         // tags start at 1

@@ -1510,11 +1510,21 @@ st_status st_nn_conv3_wgrad(const void *x, const void *dy, float *dw, int N, int
     const bf16_t *xb = static_cast<const bf16_t *>(x), *yb = static_cast<const bf16_t *>(dy);
     StreamTurn turn(s);
     const WgradTilePlan t = wgrad_tile_plan(g);
-    const WgradForm form = wgrad_form(g, t);
+    WgradForm form = wgrad_form(g, t);
+    // partial sums, or channel-major copies of both operands (slot 0); the
+    // gathering kernel where there is no room for them
+    void *ws = nullptr;
+    if (form != WG_GATHER) {
+        const st_status st = workspace_slot(0, form == WG_TILE ? (size_t)t.parts * Co * g.Kpad * sizeof(float)
+                                                               : ((size_t)g.P * Ci + (size_t)g.P * Co) * sizeof(bf16_t), s, &ws);
+        if (st == ST_ENOMEM) {
+            (void)hipGetLastError();
+            form = WG_GATHER;
+        } else if (st != ST_OK) {
+            return st;
+        }
+    }
     if (form == WG_TILE) {
-        void *ws = nullptr;
-        st_status st = workspace_slot(0, (size_t)t.parts * Co * g.Kpad * sizeof(float), s, &ws);
-        if (st != ST_OK) return st;
         float *part = static_cast<float *>(ws);
         int wide = Co % 4 == 0 && (reinterpret_cast<uintptr_t>(dy) & 7) == 0;
         void *args[] = {&xb, &yb, &part, const_cast<TileGeom *>(&t.q), const_cast<int *>(&t.ntiles), const_cast<int *>(&t.cols),
@@ -1533,10 +1543,6 @@ st_status st_nn_conv3_wgrad(const void *x, const void *dy, float *dw, int N, int
     const long long waves = nkt * nct * nch;
     const dim3 grid((unsigned)((waves + 3) / 4));
     if (form == WG_CHANNEL_MAJOR) {
-        // channel-major copies of both operands in the workspace (slot 0)
-        void *ws = nullptr;
-        st_status st = workspace_slot(0, ((size_t)g.P * Ci + (size_t)g.P * Co) * sizeof(bf16_t), s, &ws);
-        if (st != ST_OK) return st;
         bf16_t *xt = static_cast<bf16_t *>(ws), *dyt = xt + (size_t)g.P * Ci;
         const dim3 tg((unsigned)((g.P + 63) / 64));
         hipLaunchKernelGGL(k_pc_transpose, tg, dim3(256), 0, s, xb, xt, g.P, Ci);
