@@ -367,3 +367,34 @@ def test_no_room_for_workspace(host):
     try: st.dispatch_batched(problems, (), st.BATCH_PERSISTENT, stream=0x5000)
     except st.StencilError as e: assert e.status == 4  # its own table needs memory, as before
     """)
+
+
+def test_resident_poll_that_gives_up(host):
+    """A launch whose workgroups waited in vain for each other is an error of
+    the call that waits for it, or of the next one on its stream."""
+    host("""
+    def in_vain(h, n, args):  # what the kernel does: sets the word at the head of its arguments
+        word = C.cast(args[0], C.POINTER(C.POINTER(C.c_uint)))[0]
+        assert word[0] == 0
+        word[0] = 1
+        return 0
+    p = auto(64, 64, 64, iterations=24)
+    call = lambda stream, timed=False: st.dispatch_kernels(p, A, B, stream=stream, timed=timed)
+    def fails(f):
+        try: f()
+        except st.StencilError as e: return e.status == 3
+        return False
+    call(0x5000); call(0x6000)
+    answer["k_resident"] = in_vain
+    assert fails(lambda: call(0x5000, True))
+    call(0x5000)
+    answer["k_resident"] = 0
+    log.clear()
+    call(0x6000)                                     # another stream: not its failure
+    assert kernels() == ["k_resident"]
+    assert fails(lambda: call(0x5000)) and kernels() == ["k_resident"]
+    call(0x5000)                                     # reported once
+    answer["k_resident"] = in_vain
+    problems = [dict(nx=64, ny=40, nz=33, radius=1, iterations=24, op=1, u1=A, u2=B)] * 4
+    assert fails(lambda: st.dispatch_batched(problems, (), st.BATCH_PERSISTENT, stream=0x5000, timed=True))
+    """)

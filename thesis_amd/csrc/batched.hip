@@ -812,6 +812,7 @@ static st_status batch_resident(const st_problem *probs, int n, hipStream_t s, f
         st = hip_check(hipEventRecord(e1, s), "event record");
         if (st == ST_OK) st = hip_check(hipEventSynchronize(e1), "event sync");
         if (st == ST_OK) st = hip_check(hipEventElapsedTime(elapsed_ms, e0, e1), "elapsed time");
+        if (st == ST_OK) st = resident_outcome(s);
     }
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);

@@ -69,6 +69,12 @@ static thread_local const WsFixed *g_ws_fixed = nullptr;
 void workspace_use_fixed(const WsFixed *fixed) { g_ws_fixed = fixed; }
 bool workspace_is_fixed() { return g_ws_fixed != nullptr; }
 
+static const void *stream_owner(hipStream_t stream)
+{
+    static thread_local char key;
+    return stream == hipStreamPerThread ? &key : nullptr;
+}
+
 StreamTurn::StreamTurn(hipStream_t stream)
 {
     // streams that share an entry only wait for each other's launches
@@ -103,9 +109,7 @@ st_status workspace_slot(int slot, size_t bytes, hipStream_t stream, void **ptr,
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_check(e, "hipGetDevice");
     std::lock_guard<std::mutex> lock(g_ws_mutex);
-    static thread_local char thread_key;
-    const void *owner = stream == hipStreamPerThread ? &thread_key : nullptr;
-    WsBlock &w = g_ws[std::make_tuple(dev, stream, owner, slot)];
+    WsBlock &w = g_ws[std::make_tuple(dev, stream, stream_owner(stream), slot)];
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cap) != hipSuccess) (void)hipGetLastError();
     const bool capturing = cap != hipStreamCaptureStatusNone;
@@ -141,6 +145,26 @@ st_status workspace_slot(int slot, size_t bytes, hipStream_t stream, void **ptr,
     }
     w.captured |= capturing;
     *ptr = w.ptr;
+    return ST_OK;
+}
+
+st_status workspace_host_word(hipStream_t stream, bool make, unsigned **word)
+{
+    static std::map<std::tuple<int, hipStream_t, const void *>, unsigned *> words;
+    *word = nullptr;
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return hip_check(e, "hipGetDevice");
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    const auto key = std::make_tuple(dev, stream, stream_owner(stream));
+    const auto at = words.find(key);
+    if (at != words.end()) *word = at->second;
+    if (*word || !make) return ST_OK;
+    RelaxedCapture relaxed;
+    void *p = nullptr;
+    if ((e = hipHostMalloc(&p, 64, hipHostMallocDefault)) != hipSuccess) return hip_check(e, "hipHostMalloc");
+    *word = words[key] = static_cast<unsigned *>(p);
+    **word = 0;
     return ST_OK;
 }
 
@@ -468,6 +492,7 @@ st_status stencil_dispatch(const st_params *p, void *d_u1, void *d_u2, void *str
         if ((s = hip_check(hipEventRecord(e1, hs), "event record")) != ST_OK) goto done;
         if ((s = hip_check(hipEventSynchronize(e1), "event sync")) != ST_OK) goto done;
         s = hip_check(hipEventElapsedTime(elapsed_ms, e0, e1), "elapsed time");
+        if (s == ST_OK && c.resident) s = resident_outcome(hs);
     }
 done:
     if (e0) (void)hipEventDestroy(e0);

@@ -118,7 +118,10 @@ st_status run_block(const Cfg &c, void *u1, void *u2, hipStream_t s, int *in_u2)
 // registers (sweep_resident.hip), on `problems` grids of the same shape; both
 // buffers end as single sweeps leave them.  *done false: not launched (no
 // cooperative launch now, a stream under capture, or no allocation allowed).
+// A launch that waited in vain (see the kernel) fails the next run_resident on
+// its stream, or resident_outcome once the stream has been waited for.
 bool resident_eligible(const Cfg &c, int problems);
+st_status resident_outcome(hipStream_t s);
 st_status run_resident(const Cfg &c, int problems, void *const (*u)[2], hipStream_t s, bool *done);
 
 // 2D streaming temporal blocking, four or six fused sweeps per pass
@@ -160,6 +163,9 @@ private:
 // *fresh (optional) receives the block's size when this call allocated it,
 // else 0.
 st_status workspace_slot(int slot, size_t bytes, hipStream_t stream, void **ptr, size_t *fresh = nullptr);
+// A word of host memory that kernels on the stream can set, zero at first;
+// *word null where there is none yet and `make` is false.
+st_status workspace_host_word(hipStream_t stream, bool make, unsigned **word);
 constexpr int kSlotResident = 4;  // the resident form's own slot (its contents last from call to call)
 // A fixed device buffer that serves every workspace request of the calling
 // thread while it is set (one part per slot; a request larger than its

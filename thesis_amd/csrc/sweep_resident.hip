@@ -23,7 +23,8 @@
 // to launch (ctl[0], advanced by the last workgroup to finish), so what an
 // earlier launch left in a slot never matches.  All workgroups are
 // co-resident (cooperative launch, at most one per CU); a poll that finds
-// nothing for many seconds gives NaN, so every wave ends.
+// nothing for many seconds gives NaN and sets a word of host memory, so every
+// wave ends and the next call that looks at the word says so.
 //
 // Shell: sweep n reads the shell of buffer n%2, so shell cells alternate
 // between the two buffers' values: the x shell from an LDS table, shell rows
@@ -50,6 +51,7 @@ constexpr int kResPolls = 1 << 25;  // about 0.4 us each
 typedef unsigned long long ResWord;
 
 struct ResArgs {
+    unsigned *gave_up;   // host word, set by a wave whose poll found nothing
     int nx, ny, nz;
     long long sz;        // nx*ny
     int nyb, nzb;        // blocks along y and z, per problem
@@ -344,6 +346,7 @@ __global__ __launch_bounds__(64 * ROWS) void k_resident(ResArgs a, T kc)
         }
     }
     store_all((a.iters & 1) ? u1 : u0);
+    if (polls == 0 && lane == 0) __hip_atomic_store(a.gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     // the last workgroup to finish moves the tags on
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -453,6 +456,14 @@ bool resident_eligible(const Cfg &c, int problems)
     return res_pick(c, problems, device_cus()).fn != nullptr;
 }
 
+st_status resident_outcome(hipStream_t s)
+{
+    unsigned *word = nullptr;
+    if (workspace_host_word(s, false, &word) != ST_OK || !word) return ST_OK;
+    if (__atomic_exchange_n(word, 0u, __ATOMIC_RELAXED) == 0) return ST_OK;
+    return fail(ST_ELAUNCH, "an earlier dispatch on this stream waited in vain for a neighbouring workgroup: its field holds NaN");
+}
+
 st_status run_resident(const Cfg &c, int problems, void *const (*u)[2], hipStream_t s, bool *done)
 {
     *done = false;
@@ -464,7 +475,13 @@ st_status run_resident(const Cfg &c, int problems, void *const (*u)[2], hipStrea
         (void)hipGetLastError();
         return ST_OK;
     }
+    st_status st = resident_outcome(s);
+    if (st != ST_OK) return st;
     ResArgs a;
+    if (workspace_host_word(s, true, &a.gave_up) != ST_OK) {
+        (void)hipGetLastError();
+        return ST_OK;
+    }
     a.nx = c.nx; a.ny = c.ny; a.nz = c.nz;
     a.sz = (long long)c.nx * c.ny;
     a.nyb = (c.ny + k.rows - 1) / k.rows;
@@ -476,7 +493,7 @@ st_status run_resident(const Cfg &c, int problems, void *const (*u)[2], hipStrea
     const size_t bytes = head + (size_t)blocks * 2 * k.words * sizeof(ResWord);
     void *ws = nullptr;
     size_t fresh = 0;
-    st_status st = workspace_slot(kSlotResident, bytes, s, &ws, &fresh);
+    st = workspace_slot(kSlotResident, bytes, s, &ws, &fresh);
     if (st == ST_ENOMEM) {
         // no room for the faces: the caller's other form, which needs none
         (void)hipGetLastError();
