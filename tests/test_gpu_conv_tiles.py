@@ -67,3 +67,28 @@ def test_conv_tiles_infinite_neighbour(gpu):
         sees[t] = 0 <= 1 - dz < 2 and 0 <= 2 - dy < 3 and 0 <= 17 - dq < 18
     assert np.all(np.isposinf(g[:, sees, 0])) and np.all(np.isfinite(g[:, ~sees, 0]))
     assert np.all(np.isfinite(g[:, :, 1:]))
+
+
+def test_wgrad_streams_share_a_gradient(gpu):
+    """Weight gradients on several streams add up in one array: whole numbers,
+    so every order gives the same sums."""
+    st = gpu
+    from thesis_amd import nn
+    shape, ci, co = (1, 8, 8, 16), 16, 16
+    rng = np.random.default_rng(11)
+    x = rng.integers(-3, 4, shape + (ci,)).astype(np.float64)
+    gy = rng.integers(-3, 4, shape + (co,)).astype(np.float64)
+    _, want, _ = U.conv3_bwd(x, np.zeros((co, 27 * ci)), gy)
+    dx = st.DeviceArray.from_numpy(bits(x).reshape(-1, ci))
+    dg = st.DeviceArray.from_numpy(bits(gy).reshape(-1, co))
+    gw = st.DeviceArray((co, nn.kpad(ci)), np.float32)
+    gw.fill_zero()
+    streams = [st.Stream() for _ in range(4)]
+    st.synchronize()
+    print("[case] wgrad streams", flush=True)
+    for _ in range(32):
+        for s in streams:
+            nn.conv3_wgrad(dx, dg, gw, shape, ci, co, stream=s)
+    for s in streams:
+        s.sync()
+    assert np.array_equal(gw.numpy()[:, :27 * ci], 128 * want)

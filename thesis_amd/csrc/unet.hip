@@ -770,7 +770,8 @@ __global__ __launch_bounds__(64 * kWgWaves) void k_conv3_wgrad_tile(const bf16_t
 }
 
 // dW += the partial sums of all workgroups, in their order; padding columns
-// (k >= 27*Ci) are not touched
+// (k >= 27*Ci) are not touched.  One atomic per weight, so that calls on other
+// streams may add to the same gradient.
 __global__ __launch_bounds__(256) void k_wgrad_reduce(const float *__restrict__ part, float *__restrict__ dW, int n,
                                                       int K, int Kpad, int parts)
 {
@@ -786,7 +787,7 @@ __global__ __launch_bounds__(256) void k_wgrad_reduce(const float *__restrict__ 
     red[threadIdx.x] = s;
     __syncthreads();
     if (h == 0 && e < n && e % Kpad < K)
-        dW[e] += (red[threadIdx.x] + red[threadIdx.x + 64]) + (red[threadIdx.x + 128] + red[threadIdx.x + 192]);
+        atomicAdd(dW + e, (red[threadIdx.x] + red[threadIdx.x + 64]) + (red[threadIdx.x + 128] + red[threadIdx.x + 192]));
 }
 
 // ---------------------------------------------------------------- small layers
