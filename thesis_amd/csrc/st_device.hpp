@@ -13,6 +13,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+#include <utility>
+
 namespace st {
 
 enum : int { OP_THESIS = 0, OP_JACOBI = 1 };
@@ -89,6 +92,30 @@ __device__ __forceinline__ T finish_fast(T sum, T centre, T kc, bool &odd)
 }
 
 __device__ __forceinline__ bool interior1(int i, int n, int r) { return i >= r && i < n - r; }
+
+// Wave-wide DPP rotates: lane i receives the value of lane i-1 / i+1.
+template <int CTRL, typename T>
+__device__ __forceinline__ T dpp_rotate(T v)
+{
+    if constexpr (sizeof(T) == 4) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+    } else {
+        const long long b = __double_as_longlong(v);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), CTRL, 0xF, 0xF, true);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, true);
+        return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+    }
+}
+template <typename T> __device__ __forceinline__ T from_left(T v) { return dpp_rotate<0x13C>(v); }
+template <typename T> __device__ __forceinline__ T from_right(T v) { return dpp_rotate<0x134>(v); }
+
+// f(0), f(1), .. with constant arguments, until one returns false (a plain
+// unrolled loop of a march's size exceeds the unroller's limit)
+template <int... I, typename F>
+__device__ __forceinline__ void each_phase(std::integer_sequence<int, I...>, F f)
+{
+    (void)(f(std::integral_constant<int, I>{}) && ...);
+}
 
 // Cross-lane read of a 32-bit or 64-bit value from lane `src` (0..63; any
 // other value wraps modulo 64) through ds_bpermute, which needs no LDS

@@ -35,22 +35,6 @@
 
 namespace st {
 
-// wave-wide rotates: lane i receives the value of lane i-1 / i+1
-template <typename T, int CTRL>
-__device__ __forceinline__ T lane_rotate(T v)
-{
-    if constexpr (sizeof(T) == 4) {
-        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
-    } else {
-        const long long b = __double_as_longlong(v);
-        const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), CTRL, 0xF, 0xF, true);
-        const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, true);
-        return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-    }
-}
-template <typename T> __device__ __forceinline__ T from_left(T v) { return lane_rotate<T, 0x13C>(v); }
-template <typename T> __device__ __forceinline__ T from_right(T v) { return lane_rotate<T, 0x134>(v); }
-
 struct BlockArgs {
     int nx, ny;
     int tx, ty;  // blocks per axis

@@ -61,19 +61,6 @@ struct ResArgs {
     void *u[kResProblems][2];
 };
 
-template <typename T, int CTRL>
-__device__ __forceinline__ T res_rotate(T v)
-{
-    if constexpr (sizeof(T) == 4) {
-        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
-    } else {
-        const long long b = __double_as_longlong(v);
-        const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), CTRL, 0xF, 0xF, true);
-        const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, true);
-        return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-    }
-}
-
 // A face row: CX values per lane, sizeof(T)/4 words each, word i of lane l
 // at [i*64 + l].
 __device__ __forceinline__ void word_put(ResWord *p, ResWord v)
@@ -324,7 +311,7 @@ __global__ __launch_bounds__(64 * ROWS) void k_resident(ResArgs a, T kc)
                     const V m = *reinterpret_cast<const V *>(&buf[q][w][x]);
                     const V p = *reinterpret_cast<const V *>(&buf[q][w + 2][x]);
                     const T xv = xsh[slot ^ 1][w][z][xe];
-                    const T xl = res_rotate<T, 0x13C>(old[CX - 1]), xr = res_rotate<T, 0x134>(old[0]);
+                    const T xl = from_left(old[CX - 1]), xr = from_right(old[0]);
                     T sum[CX], res[CX];
 #pragma unroll
                     for (int c = 0; c < CX; ++c) {

@@ -42,26 +42,6 @@ struct RollArgs {
 template <typename T> constexpr int roll_cx() { return 16 / (int)sizeof(T); }
 __host__ __device__ constexpr int roll_halo(int r, int steps, int cx) { return (r * steps + cx - 1) / cx * cx; }
 
-template <typename T, int CTRL>
-__device__ __forceinline__ T roll_rotate(T v)
-{
-    if constexpr (sizeof(T) == 4) {
-        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
-    } else {
-        const long long b = __double_as_longlong(v);
-        const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), CTRL, 0xF, 0xF, true);
-        const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, true);
-        return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-    }
-}
-
-// f(0), f(1), .. with constant arguments, until one returns false
-template <int... I, typename F>
-__device__ __forceinline__ void roll_phases(std::integer_sequence<int, I...>, F f)
-{
-    (void)(f(std::integral_constant<int, I>{}) && ...);
-}
-
 template <int OP, int R, int STEPS, typename T>
 __global__ __launch_bounds__(256) void k_roll(const T *__restrict__ in, T *out, RollArgs a, T kc)
 {
@@ -119,7 +99,7 @@ __global__ __launch_bounds__(256) void k_roll(const T *__restrict__ in, T *out, 
     for (int i = 0; i < PF; ++i) pre[i] = row_of(rin, m_lo + i);
 
     for (int m0 = m_lo; m0 < m_hi; m0 += PH) {
-        roll_phases(std::make_integer_sequence<int, PH>{}, [&](auto phase) {
+        each_phase(std::make_integer_sequence<int, PH>{}, [&](auto phase) {
             constexpr int ph = decltype(phase)::value, rp = ph % R;
             const int m = m0 + ph;
             if (m >= m_hi) return false;
@@ -142,8 +122,8 @@ __global__ __launch_bounds__(256) void k_roll(const T *__restrict__ in, T *out, 
                 for (int k = 1; k <= NL; ++k)
 #pragma unroll
                     for (int c = 0; c < CX; ++c) {
-                        v[(NL - k) * CX + c] = roll_rotate<T, 0x13C>(v[(NL - k + 1) * CX + c]);
-                        v[(NL + k) * CX + c] = roll_rotate<T, 0x134>(v[(NL + k - 1) * CX + c]);
+                        v[(NL - k) * CX + c] = from_left(v[(NL - k + 1) * CX + c]);
+                        v[(NL + k) * CX + c] = from_right(v[(NL + k - 1) * CX + c]);
                     }
                 T s[CX], done[CX], old[CX], res[CX];
 #pragma unroll

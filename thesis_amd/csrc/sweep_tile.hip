@@ -48,7 +48,7 @@ __host__ __device__ constexpr int tile_waves(int cx) { return 32 / cx; }
 struct TileArgs {
     int nx, ny, nz;
     long long sz;            // nx*ny
-    int tx, ty, zchunk, ntiles;
+    int tx, ty, zchunk;
     const int *eq;           // 1 when both buffers' shells are equal (whole
                              // rows are stored then, shell cells unchanged)
 };
@@ -64,14 +64,6 @@ template <int R, int RY, int CX, typename T> constexpr int tile_words()
     return (tile_row_words<R, RY, T>() * tile_rows<R, RY>() + 64 * tile_waves(CX) - 1) / (64 * tile_waves(CX));
 }
 template <int R, int RY, typename T> constexpr int tile_lds() { return 2 * tile_rows<R, RY>() * tile_row_words<R, RY, T>() * 16; }
-
-// f(0), f(1), .. with constant arguments, until one returns false (a plain
-// unrolled loop of this size exceeds the unroller's limit from radius 9)
-template <int... I, typename F>
-__device__ __forceinline__ void each_phase(std::integer_sequence<int, I...>, F f)
-{
-    (void)(f(std::integral_constant<int, I>{}) && ...);
-}
 
 template <int OP, int R, int RY, int CX, bool LIGHT, typename T>
 __global__ __launch_bounds__(64 * tile_waves(CX)) void k_tile(const T *__restrict__ in, T *__restrict__ out, TileArgs a, T kc)
@@ -487,7 +479,6 @@ st_status launch_tile(const Cfg &c, const void *in, void *out, hipStream_t s)
     a.tx = (c.nx + kTileX - 1) / kTileX;
     a.ty = (c.ny + 32 * c.cy - 1) / (32 * c.cy);
     a.zchunk = c.zchunk;
-    a.ntiles = c.gx;
     a.eq = c.shell_eq;
     double kd = c.op == OP_THESIS ? (double)(2 * c.dims * c.r) : c.weight;
     float kf = (float)kd;
