@@ -30,8 +30,12 @@
  *     partials, the batch table), allocated on first use per device and
  *     stream and kept until the process ends.
  *   - Calls are stream-ordered.  Calls on different streams never share
- *     workspace; they are re-entrant for disjoint buffers and not
- *     thread-safe on the same buffers.
+ *     workspace (hipStreamPerThread counts as one per thread); they are
+ *     re-entrant for disjoint buffers and not thread-safe on the same
+ *     buffers.  What threads enqueue on one stream comes in whole calls.
+ *   - Calls that use workspace may be captured; a block that a captured
+ *     graph holds is kept until the process ends.  Where there is no memory
+ *     for one, a call takes a form that needs none if there is one.
  */
 #ifndef THESIS_AMD_STENCIL_ABI_H
 #define THESIS_AMD_STENCIL_ABI_H
@@ -170,13 +174,17 @@ typedef struct st_launch_info {
     int grid_x, grid_y, grid_z;
     int coarsen_x, coarsen_y;
     int zchunk;                  /* planes per workgroup (SMEM_REGISTER)       */
-    int temporal_steps;          /* sweeps per pass (COOP; AUTO on 2D grids,
-                                    which fuses sweeps whichever single-sweep
-                                    family `variant` names)                    */
+    int temporal_steps;          /* sweeps per pass (COOP; AUTO, which fuses
+                                    sweeps on 2D grids, and all of them on
+                                    small 3D grids of radius 1, whichever
+                                    single-sweep family `variant` names)      */
     int lds_bytes;               /* LDS per workgroup                          */
     int launches;                /* sweep-kernel launches for `iterations`
-                                    sweeps (the shell comparison and the
-                                    streaming form's band fix-ups are extra) */
+                                    sweeps (the shell comparison is extra).
+                                    AUTO's single launch of a small 3D grid
+                                    is one per sweep of the family named
+                                    under capture, in stencil_dispatch_noalloc
+                                    and where the launch is refused            */
 } st_launch_info;
 
 /* Default knobs of include/constants.h:1-52: DIM 256, DIMENSIONS 3,
@@ -208,7 +216,11 @@ st_status stencil_sweep(const st_params *p, const void *d_in, void *d_out, void 
  * intermediate state, not sweep iterations-1 (AUTO: as the family that
  * stencil_launch_config names).  If elapsed_ms is not NULL the
  * call brackets the sweep loop with HIP events on `stream`, waits for the
- * stop event and stores the time in milliseconds (host set-up excluded). */
+ * stop event and stores the time in milliseconds (host set-up excluded).
+ * In AUTO's single launch of a small 3D grid workgroups wait for each other;
+ * if one waited in vain for many seconds the field holds NaN, and the call
+ * returns ST_ELAUNCH if it waits for its own time, else the next such
+ * dispatch on the stream does. */
 st_status stencil_dispatch(const st_params *p, void *d_u1, void *d_u2, void *stream,
                            int *result_in_u2, float *elapsed_ms);
 
@@ -218,8 +230,8 @@ st_status stencil_dispatch(const st_params *p, void *d_u1, void *d_u2, void *str
  * sweeps and result as stencil_dispatch (elapsed time is not measured).  The
  * dispatch's device scratch comes from a static device array of 16 MiB +
  * 5 KiB (one per device, held until the process ends) instead of the
- * library's allocated workspace: the row form's shell flag (4 KiB part) and
- * the streaming form's shell flags and x-shell table (1 KiB + 16 B per grid
+ * library's allocated workspace: the row and tile forms' shell flag (4 KiB
+ * part) and the streaming form's shell flags and x-shell table (1 KiB + 16 B per grid
  * row: grids with ny*nz up to 2^20); a larger request fails with ST_EINVAL.
  * Calls that overlap on one device share that array and race; calls ordered
  * on one stream, or one after another, do not. */

@@ -267,21 +267,24 @@ static st_status resolve(const st_params *p, Cfg &c, bool mixed)
         //     grid-wide barrier of a cooperative launch costs 25-30 us on
         //     this device, a kernel boundary a few (512^3, 100 sweeps: 10.1 ms
         //     against 11.4 for one cooperative launch);
-        //   * it wins over the per-sweep row kernel from 320^3 up, with equal
-        //     shells (two sweeps per pass; 320^3: 1065 against 771 GCells/s)
-        //     and with different shells (one sweep per pass; 622 against
-        //     567); at 288^3 and below the row kernel, served from the
-        //     256 MiB last-level cache, wins with different shells (288^3:
-        //     660 against 554) though not with equal ones (739 against 935),
-        //     and the shells are compared on the device only, so the switch
-        //     sits between 288^3 and 320^3 (both fields above 192 MiB);
+        //   * the switch to it sits between 288^3 and 320^3 (both fields above
+        //     192 MiB), where the per-sweep kernels no longer run from the
+        //     256 MiB last-level cache.  64 sweeps, us each, streaming / row or
+        //     tile kernel, with equal and with different shells: 320^3 JACOBI
+        //     31.7 / 50.4 and 40.6 / 54.7, THESIS 39.0 / 50.3 and 66 / 56; 288^3
+        //     JACOBI 26.1 / 33.5 and 33.8 / 35.7, THESIS 32.5 / 30.2 and 54 / 35.5;
+        //     256^3 JACOBI 16.8 / 22.3 and 19.5 / 23.3, THESIS 17.2 / 19.8 and
+        //     26.7 / 24.2; 192^3 JACOBI 10.1 / 12.2 and 12.4 / 12.8, THESIS 10.9 /
+        //     12.0 and 17.8 / 13.9.  JACOBI alone would put it lower;
         //   * grids of up to about a million cells (3D) or four million (2D)
         //     are bound by the launch cadence, where the plain kernel is the
-        //     cheapest (64^3: 2.5 us against 5.2 for the row kernel and 8.3
-        //     for the streaming form; 256^2: 2.5 against 7.5 for the 2D
-        //     register march);
-        //   * elsewhere the register march / row kernel wherever it is
-        //     instantiated, else the plain kernel.
+        //     cheapest per-sweep one (64^3: 2.5 us against 5.2 for the row
+        //     kernel and 8.3 for the streaming form; 256^2: 2.5 against 7.5
+        //     for the 2D register march);
+        //   * elsewhere the SMEM_REGISTER forms wherever they are ahead of it.
+        // These name the family (stencil_sweep, stencil_launch_config); what
+        // a dispatch of a 2D grid or of a small 3D grid of radius 1 runs
+        // instead is decided further down.
         c.bx = c.by = c.bz = 0;
         c.heuristic = 1;
         const long long cells = (long long)c.nx * c.ny * c.nz;
@@ -297,9 +300,7 @@ static st_status resolve(const st_params *p, Cfg &c, bool mixed)
         } else if (c.dims == 2 && c.iters >= 8 && c.form == 0 && (c.tsteps == 0 || c.tsteps == 4 || c.tsteps == 6) &&
                    stream2d_eligible(c) && cells >= small) {
             // 2D beyond the launch-bound sizes: six or four fused sweeps per
-            // pass (64 sweeps: 4096^2 1511 GCells/s against 771 for the
-            // register march, 2048^2 570 against 404 for the plain kernel;
-            // 1024^2 stays with the plain kernel, 212 against 143)
+            // pass, run as such from 2^29 cells (below, the block form)
             c.variant = ST_V_COOP;
             c.cx = 1;
             c.cy = 0;

@@ -3,7 +3,7 @@
 // harnesses that forbid hipMalloc).  No reference counterpart.
 //
 // The dispatch's own device scratch lives in the file-scope array `scratch`
-// below instead of the library's allocated workspace: the row form's
+// below instead of the library's allocated workspace: the row and tile forms'
 // shell-comparison flag (slot 2, 4 KiB part) and the streaming form's flags
 // and x-shell table of both buffers (slot 3: 1 KiB + 16 B per row of the
 // grid, a 16 MiB + 1 KiB part, so grids with ny*nz up to 2^20 rows).  Each

@@ -25,7 +25,7 @@
 // sweeps about 7), above that the VALU: a block computes every row at every
 // level, 64*32 cells for (64-2*steps)*(32-2*steps) stored.  64 sweeps, FP32
 // JACOBI, before (plain kernel below 2048^2, streaming form above) and now:
-// 256^2 172 -> 61 us, 1024^2 322 -> 100, 2048^2 452 -> 178, 4096^2 696 ->
+// 256^2 172 -> 59 us, 1024^2 322 -> 100, 2048^2 452 -> 178, 4096^2 696 ->
 // 408, 16384^2 6.00 -> 5.26 ms; different shells, which the streaming form
 // sweeps singly, 4096^2 THESIS 1946 -> 552 us.
 #include <algorithm>

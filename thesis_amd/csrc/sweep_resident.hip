@@ -17,7 +17,7 @@
 // the number of the sweep it belongs to, in relaxed agent-scope atomics.  A
 // reader polls the word itself until the tag is the one it needs, so there
 // is no flag, no fence and no grid barrier (a cooperative grid barrier costs
-// 25 us here, a hop of this exchange about 0.4).  Two slots alternate: a wave
+// 25 us here, a hop of this exchange about 0.4, a round trip 0.8).  Two slots alternate: a wave
 // sends sweep n+2 only after it has its neighbour's words of sweep n+1, which
 // the neighbour sends after reading those of sweep n.  Tags go on from launch
 // to launch (ctl[0], advanced by the last workgroup to finish), so what an
@@ -128,7 +128,7 @@ constexpr int res_stage()
 }
 
 // words of one block's incoming faces of one slot: rows [0, NZ) below,
-// [NZ, 2*NZ) above in y; [2*NZ, +16) below, [.., +16) above in z
+// [NZ, 2*NZ) above in y; [2*NZ, +ROWS) below, [.., +ROWS) above in z
 template <int ROWS, int CX, int NZ, typename T>
 constexpr long long res_face_words() { return (2LL * NZ + 2 * ROWS) * 64 * CX * (sizeof(T) / 4); }
 
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(64 * ROWS) void k_resident(ResArgs a, T kc)
     constexpr int ZS = res_stage<CX, NZ, T>(), NS = NZ / ZS;
     constexpr int RW = 64 * CX * (int)(sizeof(T) / 4);  // words of a face row
     typedef T V __attribute__((ext_vector_type(CX)));
-    __shared__ __align__(16) T rows[2][ZS][ROWS + 2][64 * CX];  // row w at [w + 1]; [0], [17]: halo
+    __shared__ __align__(16) T rows[2][ZS][ROWS + 2][64 * CX];  // row w at [w + 1]; [0], [ROWS + 1]: halo
     __shared__ T xsh[2][ROWS][NZ][2];                           // columns 0 and nx-1 of each buffer
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
