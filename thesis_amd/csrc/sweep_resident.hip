@@ -140,6 +140,16 @@ __global__ __launch_bounds__(64 * ROWS) void k_resident(ResArgs a, T kc)
     typedef T V __attribute__((ext_vector_type(CX)));
     __shared__ __align__(16) T rows[2][ZS][ROWS + 2][64 * CX];  // row w at [w + 1]; [0], [ROWS + 1]: halo
     __shared__ T xsh[2][ROWS][NZ][2];                           // columns 0 and nx-1 of each buffer
+    // Whether a poll of this workgroup gave up.  Where FP32 state fills the
+    // registers a word of LDS holds it: `polls` outliving the sweeps would
+    // spill (148x231x93 9% slower); elsewhere `polls` does, the LDS word
+    // costing up to 26% (36x430x105 FP64).
+    constexpr bool kWord = sizeof(T) == 4 && CX * NZ >= (ROWS == 16 ? 32 : 64);
+    __shared__ int gave_up;
+    if constexpr (kWord) {
+        if (threadIdx.x == 0) gave_up = 0;
+        __syncthreads();
+    }
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int per = a.nyb * a.nzb;
@@ -266,6 +276,7 @@ __global__ __launch_bounds__(64 * ROWS) void k_resident(ResArgs a, T kc)
                 for (int left = polls; !fy.here(tag); fy.load(row, lane))
                     if (--left < 0) {
                         polls = 0;
+                        if constexpr (kWord) gave_up = 1;
                         break;
                     }
                 T h[CX];
@@ -289,6 +300,7 @@ __global__ __launch_bounds__(64 * ROWS) void k_resident(ResArgs a, T kc)
                 if (all) break;
                 if (--left < 0) {
                     polls = 0;
+                    if constexpr (kWord) gave_up = 1;
                     break;
                 }
             }
@@ -333,10 +345,15 @@ __global__ __launch_bounds__(64 * ROWS) void k_resident(ResArgs a, T kc)
         }
     }
     store_all((a.iters & 1) ? u1 : u0);
-    if (polls == 0 && lane == 0) __hip_atomic_store(a.gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if constexpr (!kWord) {
+        if (polls == 0 && lane == 0) __hip_atomic_store(a.gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     // the last workgroup to finish moves the tags on
     __syncthreads();
     if (threadIdx.x == 0) {
+        if constexpr (kWord) {
+            if (gave_up) __hip_atomic_store(a.gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
         const unsigned d = __hip_atomic_fetch_add(a.ctl + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (d == gridDim.x - 1) {
             __hip_atomic_store(a.ctl + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
