@@ -81,11 +81,12 @@ def test_conv_forms(host):
         nn.conv3(A, A, A, A, None, shape, ci, co)
         return kernels()
     for shape, ci, co in (((8, 64, 64, 64), 48, 16), ((8, 64, 64, 64), 16, 48), ((8, 16, 16, 16), 64, 64),
-                          ((8, 32, 32, 32), 96, 32), ((8, 32, 32, 32), 64, 64), ((4, 4, 4, 4), 16, 16), ((1, 2, 2, 2), 8, 16)):
+                          ((8, 32, 32, 32), 96, 32), ((8, 32, 32, 32), 64, 64), ((4, 4, 4, 4), 16, 16), ((1, 2, 2, 2), 8, 16),
+                          ((8, 8, 1, 60), 40, 40), ((6, 9, 1, 21), 32, 52)):
         assert route(shape, ci, co) == ["k_conv3_tile"], (shape, ci, co)
     for shape, ci, co in (((1, 1, 1, 100000), 16, 16), ((1, 300, 300, 3), 64, 64), ((4, 20, 20, 20), 128, 128),
                           ((1, 40, 40, 40), 64, 80), ((8, 32, 32, 32), 64, 80), ((64, 8, 8, 8), 64, 256),
-                          ((4000, 2, 2, 2), 8, 16), ((1, 1, 300, 301), 32, 32)):
+                          ((4000, 2, 2, 2), 8, 16), ((1, 1, 300, 301), 32, 32), ((7, 13, 34, 63), 80, 96)):
         assert route(shape, ci, co) == ["k_conv3"], (shape, ci, co)
     """)
 

@@ -1344,11 +1344,11 @@ static int conv_flat_nb(int co) { return co >= 64 ? 4 : (co >= 32 ? 2 : 1); }
 
 // Whether the tiles are ahead of k_conv3, by the time a chunk of 32 weight
 // columns takes in each (us, fitted to 690 shapes of 8 to 262144 positions and
-// 4 to 256 channels; the choice is within 1% of the better one on average, at
-// worst 1.2 times).  Tiles: per round of workgroups, by channel blocks, depth
+// 4 to 256 channels; there and on 417 random shapes the choice is within 0.3%
+// of the better one on average, at worst 1.3 times).  Tiles: per round of workgroups, by channel blocks, depth
 // and workgroups per CU.  k_conv3: a latency until the waves fill the card,
 // then a rate; taps outside a sample of one plane, row or column cost it no
-// load.  64 -> 64 channels, tiles / k_conv3: 8 x 16^3 31 / 64, 1 x 40^3
+// load, which shows once there are waves enough.  64 -> 64 channels, tiles / k_conv3: 8 x 16^3 31 / 64, 1 x 40^3
 // 83 / 69; 64 -> 80 (channel blocks in two halves, each staging the tile)
 // 135 / 91; 1 x 300 x 300 x 3 (3 of 16 columns) 1136 / 232.
 static bool conv_tile_ahead(const ConvGeom &g, int nb, int mb, bool two_per_cu, int blocks)
@@ -1358,9 +1358,11 @@ static bool conv_tile_ahead(const ConvGeom &g, int nb, int mb, bool two_per_cu, 
     double t = (double)((blocks + round - 1) / round) * tile[nb - 1][mb == 4 || (nb == 4 && two_per_cu)];
     if ((g.Co + 15) / 16 % nb) t *= 1.2;  // a last group of fewer blocks
     const int fb = conv_flat_nb(g.Co);
-    const double waves = (double)((g.P + 63) / 64) * ((g.Co + 16 * fb - 1) / (16 * fb)) / 1024;
+    // in 1024; of four channel blocks, those with fewer as their share
+    const double groups = fb == 4 ? (g.Co + 15) / 16 / 4.0 : (g.Co + 16 * fb - 1) / (16 * fb);
+    const double waves = (double)((g.P + 63) / 64) * groups / 1024;
     double f = fb == 1 ? std::max(0.95, 0.50 * waves) : fb == 2 ? std::max(0.85, 0.60 * waves) : std::max(1.15, 0.87 * waves);
-    if (g.D == 1 || g.H == 1 || g.W == 1) f *= 0.7;
+    if (waves >= 0.25 && (g.D == 1 || g.H == 1 || g.W == 1)) f *= 0.7;
     return t <= f;
 }
 
