@@ -66,7 +66,8 @@ def test_wgrad_forms(host):
     assert route((1, 1, 1, 100000), 64, 64) == ROWS       # 1 of 16 rows of a tile, whole octets of positions
     assert route((1, 20000, 1, 1), 64, 64) == GATHER      # 1 of 64 positions
     assert route((1, 20000, 1, 1), 16, 16) == TILE
-    assert route((1, 2, 2, 8), 64, 64) == GATHER
+    assert route((1, 2, 2, 8), 64, 64) == GATHER and route((8, 4, 4, 1), 152, 120) == GATHER
+    assert route((1, 4, 4, 4), 16, 16) == TILE and route((4, 4, 4, 4), 64, 64) == TILE
     assert route((1, 1, 1, 1000), 64, 64) == TILE
     assert route((8, 16, 16, 16), 192, 32) == GATHER      # no tile fits
     """)

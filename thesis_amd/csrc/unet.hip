@@ -1463,7 +1463,13 @@ static WgradForm wgrad_form(const ConvGeom &g, const WgradTilePlan &t)
     const bool rows = g.W % 8 == 0 && g.Ci <= kTrMaxC && g.Co <= kTrMaxC;
     const WgradForm flat = rows ? WG_CHANNEL_MAJOR : WG_GATHER;
     if (!t.fn) return flat;
-    if (g.P <= (g.Ci >= 32 ? 64 : 32)) return WG_GATHER;
+    // up to 256 positions: a step of the gathering kernel per 32, against the
+    // columns of a wave and the reduction (us; within 3 of the measured times)
+    if (g.P <= 256) {
+        const double gather = 3.5 + 4.6 * ((g.P + 31) / 32);
+        const double tile = 8 + 0.7 * ((t.cols + kWgWaves - 1) / kWgWaves) + t.parts * 2e-6 * g.Co * g.Kpad;
+        if (gather < tile) return WG_GATHER;
+    }
     const long long room = (long long)t.ntiles * t.positions, P = g.P;
     // rows of positions alone: 18 of 27 taps lie outside and cost no load
     const int least = rows || (g.D == 1 && g.H == 1) ? 8 : 16;
