@@ -221,7 +221,7 @@ def test_small_interiors(host):
         log.clear()
         st.dispatch_kernels(auto(nx, ny, nz, radius=r, dtype=dt, iterations=2), A, B)
         return kernels()[-1]
-    march = {(1000, 33, 33): (6, 8), (4000, 20, 20): (6, 8), (40, 4000, 20): (8,), (9, 9, 100000): (1,)}
+    march = {(1000, 33, 33): (6, 8), (4000, 20, 20): (6, 8), (40, 4000, 20): (8,), (90, 548, 34): (8,), (9, 9, 100000): (1,)}
     plain = {(1000, 33, 33): (10, 12), (104, 104, 104): (10, 12), (33, 33, 2000): (12,), (33, 33, 5000): (16,)}
     plain64 = {(1000, 33, 33): (5, 6, 8), (4000, 20, 20): (5, 6, 8), (33, 33, 2000): (10,), (12000, 12000, 11): (5,)}
     tile = {(1000, 33, 33): (2, 4), (1000, 1000, 20): (6, 8), (2000, 500, 24): (10,), (104, 104, 104): (6, 8), (64, 64, 400): (12,),

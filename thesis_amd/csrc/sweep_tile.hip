@@ -377,8 +377,8 @@ static bool tile_light(const Cfg &c, int ch) { return tile_cx(c) == 2 || tile_wo
 //   * a tile computes shell cells like any other and marches through 2R planes
 //     of halo: FP32 radii 6 to 8 stay with the register march where little of
 //     the grid is interior (1000x33x33 R = 8 11 / 16.5, R = 6 10.9 / 14), up to
-//     a larger size where that has fewer planes than the halo (40x4000x20
-//     R = 8 10 / 12.6, 1000x1000x20 R = 6 40 / 25.5), and radius 1 where 15/16 of
+//     a larger size where that is few planes beside the halo (40x4000x20
+//     R = 8 10 / 12.6, 90x548x34 15 / 17.5, 1000x1000x20 R = 6 40 / 25.5), and radius 1 where 15/16 of
 //     the tiles lie outside (9x9x100000 93 / 118).
 static long long ceil_to(long long n, long long unit) { return (n + unit - 1) / unit * unit; }
 
@@ -401,7 +401,7 @@ bool tile_eligible(const Cfg &c)
     if (c.r <= 4 && c.nx % 4 == 0 && (rows_consecutive(c) || (c.nx > 512 && c.r <= (es == 8 ? 2 : 1))))
         return false;
     if (c.r == 1 && 16 * cells < tiles_rounded(c)) return false;
-    if (es == 4 && c.r >= 6 && c.r <= 8 && interior_rounded(c) < (c.nz < 4 * c.r ? 3LL << 20 : 5LL << 17)) return false;
+    if (es == 4 && c.r >= 6 && c.r <= 8 && interior_rounded(c) < (c.nz < 5 * c.r ? 3LL << 20 : 1LL << 19)) return false;
     return tile_kernel_for(c, 1, tile_cx(c), true).fn != nullptr;
 }
 
@@ -411,7 +411,9 @@ bool tile_eligible(const Cfg &c)
 // 7 / 19, 104^3 R = 12 18 / 20, 128^3 R = 12 31 / 21; FP64 1000x33x33 R = 8 9.7 /
 // 19.6, 4000x20x20 R = 6 12.6 / 14.3, 104^3 R = 8 29 / 21), and where the slower
 // kernels of wide stars spend themselves on shell cells (33x33x2000 FP64 R = 10
-// 48 / 93, FP32 R = 12 30 / 37; 2000x500x24 FP64 R = 10 148 / 121).
+// 48 / 93, FP32 R = 12 30 / 37; 2000x500x24 FP64 R = 10 148 / 121).  Between
+// 3 << 17 and 7 << 17 interior cells FP32 goes either way (235x30x175 R = 10 20 /
+// 15, 457x34x95 12 / 19).
 bool tile_over_plain(const Cfg &c)
 {
     const long long in = interior_rounded(c), all = tiles_rounded(c);
