@@ -297,6 +297,15 @@ def test_mixed_precision_vs_oracle(gpu, oracle, dtype, dims, shape, r):
     assert_bitwise(du.numpy(), want, f"mixed {dtype}")
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("dims,shape,r", [
+    # interiors of 1, 64 and 65 columns, 1 to 5 rows, small and beyond 2^18 lanes
+    (2, (17, 300, 1), 8), (2, (80, 19, 1), 8), (2, (81, 21, 1), 8), (2, (73, 13, 1), 4), (3, (17, 18, 20), 8),
+    (3, (65, 21, 22), 10), (2, (1041, 530, 1), 9), (3, (130, 75, 71), 1), (3, (131, 75, 71), 2), (3, (71, 90, 75), 7)], ids=str)
+def test_mixed_lane_kernels(gpu, oracle, dtype, dims, shape, r):
+    test_mixed_precision_vs_oracle(gpu, oracle, dtype, dims, shape, r)
+
+
 @pytest.mark.parametrize("its", [1, 2, 3, 7, 10, 11])
 @pytest.mark.parametrize("tsteps", [2, 3, 4])
 def test_coop_pass_schedule(gpu, oracle, its, tsteps):

@@ -104,6 +104,25 @@ def test_mixed_small_kernels(host):
     """)
 
 
+def test_mixed_lane_kernels(host):
+    """64 x 4 threads per workgroup where the grid is small or its rows fill the
+    wavefronts, the flat kernels elsewhere."""
+    host("""
+    def route(dims, nx, ny, nz, radius):
+        log.clear()
+        p = st.StencilParams.make(nx=nx, ny=ny, nz=nz, dimensions=dims, radius=radius, op=1, dtype=st.BF16,
+                                  iterations=3, restart=10)
+        st.dispatch_mixed(p, A, A, A, A, A)
+        return [k.split("<")[0] for k in kernels() if "sweep" in k or "defect" in k]
+    for call in ((3, 256, 256, 256, 8), (3, 123, 284, 71, 1), (3, 123, 284, 71, 2), (2, 2048, 2048, 1, 16),
+                 (3, 41, 41, 41, 5), (2, 88, 2912, 1, 8), (2, 59, 202, 1, 14), (3, 114, 99, 104, 10)):
+        assert route(*call) == ["k_mx_defect_rows"] + ["k_mx_sweep_rows"] * 3, (call, kernels())
+    for call in ((3, 123, 284, 71, 3), (3, 333, 251, 207, 6), (3, 70, 70, 70, 2), (3, 67, 123, 194, 1), (3, 97, 50, 351, 14),
+                 (2, 11, 100000, 1, 4), (2, 41, 3001, 1, 5), (2, 2048, 2048, 1, 5)):
+        assert route(*call) == ["k_mx_defect"] + ["k_mx_sweep"] * 3, (call, kernels())
+    """)
+
+
 def test_layer_grids(host):
     """Workgroups of the layers that move bytes follow the groups of channels,
     whatever the shape; a loss over many values takes more blocks."""

@@ -10,6 +10,8 @@
 // Every `restart` sweeps the correction is folded into x in FP32 and the
 // defect is recomputed in FP32 from the new x (the FP32-residual defect
 // correction); 16-bit rounding then only ever applies to increments.
+#include <algorithm>
+
 #include "st_device.hpp"
 #include "st_half.hpp"
 #include "st_internal.hpp"
@@ -93,6 +95,110 @@ __global__ __launch_bounds__(256) void k_mx_sweep(const uint16_t *__restrict__ e
     }
 }
 
+// The same with 64 columns x 4 rows of threads per workgroup, so that a cell is
+// found without the divisions of a flat index, and the sums of radius 1 and 2
+// unrolled (RS; 0: any radius).  Bound: the 2-byte loads of a cell's 4R or 6R
+// neighbours, one instruction each.  f(index) for every interior cell.
+template <typename F>
+__device__ __forceinline__ void each_interior(const MixArgs &a, F f)
+{
+    const Geom &g = a.g;
+    const int R = g.r, k0 = a.dims == 3 ? R : 0, k1 = a.dims == 3 ? g.nz - R : 1;
+    for (int k = k0 + (int)blockIdx.z; k < k1; k += (int)gridDim.z)
+        for (long long j = R + (long long)blockIdx.y * 4 + (threadIdx.x >> 6); j < g.ny - R; j += 4LL * gridDim.y)
+            for (long long i = R + (long long)blockIdx.x * 64 + (threadIdx.x & 63); i < g.nx - R; i += 64LL * gridDim.x)
+                f(i + j * g.sy + k * g.sz);
+}
+
+// Sum of the neighbours of p[0] in the reference's order, v(neighbour) each.
+template <int RS, typename T, typename V>
+__device__ __forceinline__ float neighbour_sum(const T *p, const MixArgs &a, V v)
+{
+    const int R = RS ? RS : a.g.r;
+    float s = 0.0f;
+    auto axis = [&](long long st) {
+#pragma unroll
+        for (int q = R; q >= 1; --q) s += v(p[-q * st]);
+#pragma unroll
+        for (int q = 1; q <= R; ++q) s += v(p[q * st]);
+    };
+    axis(1);
+    axis(a.g.sy);
+    if (a.dims == 3) axis(a.g.sz);
+    return s;
+}
+
+template <bool F16, int RS>
+__global__ __launch_bounds__(256) void k_mx_defect_rows(const float *__restrict__ x, uint16_t *__restrict__ d, MixArgs a)
+{
+    each_interior(a, [&](long long idx) {
+        const float tcell = neighbour_sum<RS>(x + idx, a, [](float q) { return q; }) * a.w;
+        d[idx] = rnd16<F16>(tcell - x[idx]);
+    });
+}
+
+template <bool F16, int RS>
+__global__ __launch_bounds__(256) void k_mx_sweep_rows(const uint16_t *__restrict__ e, const uint16_t *__restrict__ d,
+                                                       uint16_t *__restrict__ eo, MixArgs a)
+{
+    each_interior(a, [&](long long idx) {
+        const float sw = neighbour_sum<RS>(e + idx, a, [](uint16_t q) { return wid16<F16>(q); }) * a.w;
+        eo[idx] = rnd16<F16>(wid16<F16>(d[idx]) + sw);
+    });
+}
+
+// Whether the kernels with 64 x 4 threads per workgroup take the grid.  20
+// sweeps with their passes, us, flat / 64 x 4:
+// * a grid that is all in flight at once (2^18 lanes) has only its chain of
+//   loads to wait for, and lanes without a cell cost nothing: 41^3 R = 5 161 /
+//   129, R = 8 214 / 124, 99 x 270 R = 7 162 / 131, 59 x 202 R = 14 219 / 157.
+//   Not for R = 3, nor for flat rows that are half empty with few loads to
+//   save (41 x 3001 R = 5 123 / 137, R = 9 160 / 129);
+// * beyond it the time is the loads' and an empty lane costs its share.  R = 1:
+//   123 x 284 x 71 399 / 298, 67 columns (51 % filled) 298 / 330.  R = 2: 542 /
+//   454, 70^3 (52 %) 150 / 180.  R = 3 to 7, whose sums are not unrolled in
+//   eights: flat is ahead (333 x 251 x 207 R = 6 6481 / 8726, 123 x 284 x 71
+//   R = 7 973 / 1192).  From 8: 256^3 R = 8 7805 / 3657, R = 12 10137 / 5959,
+//   2048^2 R = 16 2579 / 1430, 114 x 99 x 104 R = 10 (73 %) 582 / 452; 97 x 50 x
+//   351 R = 14 (54 %) 512 / 759, 100 x 5000 R = 15 (55 %) 331 / 381.  Whole
+//   eights in 2D stay ahead down to a third: 88 x 2912 R = 8 197 / 137.  Odd
+//   radii gain less: 123 x 284 x 71 R = 15 (73 %) 934 / 1099, 700^2 R = 11 259 /
+//   304, 1031 x 1021 R = 11 506 / 370.
+static bool mx_rows(const MixArgs &a, long long w, long long wy, long long wz)
+{
+    const int R = a.g.r;
+    const long long lanes = (w + 63) / 64 * 64;
+    const long long all = lanes * wy * wz;
+    if (all <= 1 << 18 && R != 3 && (a.dims == 3 || R >= 8 || 2 * w >= lanes)) return true;
+    if ((R > 2 && R < 8) || (R > 8 && R % 2 && a.dims == 2 && all < 1 << 19)) return false;
+    return 100 * w >= (R == 1 ? 60 : R == 2 ? 80 : a.dims == 2 && R % 8 == 0 ? 35 : R % 2 ? 75 : 67) * lanes;
+}
+
+// The defect of x, or where x is null the sweep e -> eo.
+template <bool F16>
+static void mx_cells(const MixArgs &a, const float *x, const uint16_t *e, uint16_t *d, uint16_t *eo, hipStream_t s)
+{
+    auto blocks = [](long long n, long long per, long long most) { return (unsigned)std::max(1LL, std::min((n + per - 1) / per, most)); };
+    const int R = a.g.r;
+    const long long wx = a.g.nx - 2 * R, wy = a.g.ny - 2 * R, wz = a.dims == 3 ? a.g.nz - 2 * R : 1;
+    if (!mx_rows(a, wx, wy, wz)) {
+        const dim3 grid(blocks(wx * wy * wz, 256, 32768));
+        if (x) hipLaunchKernelGGL(k_mx_defect<F16>, grid, dim3(256), 0, s, x, d, a);
+        else hipLaunchKernelGGL(k_mx_sweep<F16>, grid, dim3(256), 0, s, e, d, eo, a);
+        return;
+    }
+    const unsigned bx = blocks(wx, 64, 1024), by = blocks(wy, 4, 8192);
+    const dim3 grid(bx, by, blocks(wz, 1, std::min(65535LL, (1LL << 23) / ((long long)bx * by))));   // 2^31 lanes in all
+    auto launch = [&](auto rs) {
+        constexpr int RS = decltype(rs)::value;
+        if (x) hipLaunchKernelGGL((k_mx_defect_rows<F16, RS>), grid, dim3(256), 0, s, x, d, a);
+        else hipLaunchKernelGGL((k_mx_sweep_rows<F16, RS>), grid, dim3(256), 0, s, e, d, eo, a);
+    };
+    if (R == 1) launch(std::integral_constant<int, 1>{});
+    else if (R == 2) launch(std::integral_constant<int, 2>{});
+    else launch(std::integral_constant<int, 0>{});
+}
+
 // u's shell <- x's (3D, fewer than 2^31 shell cells; the whole field took
 // 103 us of 384^3)
 __global__ __launch_bounds__(256) void k_mx_shell(const float *__restrict__ x, float *__restrict__ u, int nx, int ny, int nz,
@@ -156,8 +262,6 @@ static st_status mixed_impl(const Cfg &c, float *x, uint16_t *e1, uint16_t *e2, 
     a.dims = c.dims;
     a.w = (float)c.weight;
     const long long n = (long long)c.nx * c.ny * c.nz;
-    const int R = c.r;
-    const long long ni = (long long)(c.nx - 2 * R) * (c.ny - 2 * R) * (c.dims == 3 ? c.nz - 2 * R : 1);
     auto blocks = [](long long cnt) {
         long long b = (cnt + 255) / 256;
         if (b > 32768) b = 32768;
@@ -205,11 +309,11 @@ static st_status mixed_impl(const Cfg &c, float *x, uint16_t *e1, uint16_t *e2, 
     }
     auto defect = [&]() {
         if (rows) st = launch_rows_mixed(c, 1, F16, x, d, nullptr, s);
-        else hipLaunchKernelGGL(k_mx_defect<F16>, blocks(ni), dim3(256), 0, s, x, d, a);
+        else mx_cells<F16>(a, x, nullptr, d, nullptr, s);
     };
     auto sweep = [&](const uint16_t *ein, uint16_t *eout) {
         if (rows) st = launch_rows_mixed(c, 0, F16, ein, eout, d, s);
-        else hipLaunchKernelGGL(k_mx_sweep<F16>, blocks(ni), dim3(256), 0, s, ein, d, eout, a);
+        else mx_cells<F16>(a, nullptr, ein, d, eout, s);
     };
     defect();
     uint16_t *ea = e1, *eb = e2;
